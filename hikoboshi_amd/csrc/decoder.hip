@@ -472,7 +472,8 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   // logits weights (32 outputs, 21 used) as fp32, [k / 4][v][k % 4]: lane v reads four k of its column at once
   __shared__ __attribute__((aligned(16))) float wlg[kH * 32];
   __shared__ __attribute__((aligned(16))) float prm[kPrmSize];
-  __shared__ __attribute__((aligned(16))) float gtab[kGeluPolyLds];  // GELU polynomials
+  // GELU polynomials of the fp32 mode's FFN
+  __shared__ __attribute__((aligned(16))) float gtab[PREC == kPrecFp32 ? kGeluPolyLds : 4];
   // neighbour words of the step records: -1 for an empty slot, else j | 2^30 if j is decoded before the step
   __shared__ __attribute__((aligned(16))) int nbw[G * kKmax];
   __shared__ int cls[G * kKmax];  // layer-0 table row of each slot (with a.l0tab)
@@ -532,7 +533,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   const uint64_t seed = a.seeds[b];
   const float T = (a.temperature > 0.0F && isfinite(a.temperature)) ? a.temperature : 1.0F;
   const bool greedy = a.greedy || a.temperature <= 0.0F;
-  load_gelu_poly(gtab, threadIdx.x, kThreads);
+  if constexpr (PREC == kPrecFp32) load_gelu_poly(gtab, threadIdx.x, kThreads);
   if (threadIdx.x == 0) bad = 0;
   for (int l = 0; l < kLayers; ++l) {
     const DecLayerDev& w = m.dec[l];
@@ -850,8 +851,8 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
                   xv.y += ev.y + zv.y;
                   xv.z += ev.z + zv.z;
                   xv.w += ev.w + zv.w;
-                  float4 v = make_float4(gelu_poly(xv.x, gtab), gelu_poly(xv.y, gtab), gelu_poly(xv.z, gtab),
-                                         gelu_poly(xv.w, gtab));
+                  float4 v = make_float4(gelu_exp2(xv.x), gelu_exp2(xv.y), gelu_exp2(xv.z),
+                                         gelu_exp2(xv.w));
                   if (k >= K) v = make_float4(0.F, 0.F, 0.F, 0.F);
                   _Float16* gh = G16 + ((kPipe ? i : (s / 3) * 2) * kKmax + k) * kLdH + c;  // 16-bit: slot = member
                   const float vv[4] = {v.x, v.y, v.z, v.w};
@@ -956,7 +957,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   const int row = mb * 16 + 4 * g + e;
-                  const float gv = gelu_poly(acc[mb][e] + b2, gtab);
+                  const float gv = gelu_exp2(acc[mb][e] + b2);
                   sum += row < K ? gv : 0.0F;
                 }
               sum += __shfl_xor(sum, 16, 64);
@@ -1025,7 +1026,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
           __syncthreads();
           for (int task = threadIdx.x; task < ml * kFF; task += kThreads) {
             const int o = task % kFF;
-            const float f = gelu_poly(ys[task] + pl[kPrmBin + o], gtab);
+            const float f = gelu_exp2(ys[task] + pl[kPrmBin + o]);
             ff[task] = f;
             put_split16<PREC>(ffs16 + task, G * kFF, f);
           }
@@ -1363,7 +1364,6 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
   __shared__ __attribute__((aligned(16))) float qs[kTabSlots * kH];          // Q^0_j
   __shared__ __attribute__((aligned(16))) float ts[kV * kH];                 // T_0
   __shared__ __attribute__((aligned(16))) float hA[kH];
-  __shared__ __attribute__((aligned(16))) float gtab[kGeluPolyLds];
   __shared__ int js[kTabSlots];
   __shared__ int srows[kKmax + 1];  // rows of each slot of t, then (thread 0) their running start
   __shared__ int16_t rslot[kTabSlots * kL0Classes], rcls[kTabSlots * kL0Classes];  // row -> (slot, state)
@@ -1372,7 +1372,6 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
   const int nk = min(kTabSlots, K - k0);
   if (t >= L || nk <= 0) return;
   const DecLayerDev& w = m.dec[0];
-  load_gelu_poly(gtab, threadIdx.x, kThreads);
   for (int i = threadIdx.x; i < kH; i += kThreads) hA[i] = Q[((size_t)3 * L + t) * kH + i] + w.b1[i];
   if (threadIdx.x < nk) {
     const int jj = idx[(size_t)t * K + k0 + threadIdx.x];
@@ -1444,10 +1443,10 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
         xv.y += e.y + z.y;
         xv.z += e.z + z.z;
         xv.w += e.w + z.w;
-        vv[0] = gelu_poly(xv.x, gtab);
-        vv[1] = gelu_poly(xv.y, gtab);
-        vv[2] = gelu_poly(xv.z, gtab);
-        vv[3] = gelu_poly(xv.w, gtab);
+        vv[0] = gelu_exp2(xv.x);
+        vv[1] = gelu_exp2(xv.y);
+        vv[2] = gelu_exp2(xv.z);
+        vv[3] = gelu_exp2(xv.w);
       }
       half4 hv, lv;
 #pragma unroll
@@ -1484,7 +1483,7 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
       for (int e = 0; e < 4; ++e) {
         const int row = r0 + mb * 16 + 4 * g + e;
         const float v = acc[mb][e] + cor[mb][e] * (1.0F / 2048.0F);
-        if (row < rows) out[(size_t)row * kH + col] = gelu_poly(v + b2, gtab);
+        if (row < rows) out[(size_t)row * kH + col] = gelu_exp2(v + b2);
       }
     __syncthreads();
   }
@@ -1568,7 +1567,6 @@ __global__ __launch_bounds__(256) void rows_gemm_kernel(const float* __restrict_
   }
   __syncthreads();
   floatx4 acc[4][2];
-  zero_acc(acc);
   mfma_tile<4, 2>(A, kLd, Wp, N, cblk * kH + wave * 32, kH, acc);
   float* o = out ? out + (size_t)cblk * M * kH : nullptr;
   _Float16* oh = (out_h && cblk < nh) ? out_h + (size_t)cblk * M * kH : nullptr;

@@ -59,7 +59,6 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * kRows * kLdS1];
   float* A = reinterpret_cast<float*>(S);
   static_assert(kRows * kLd * sizeof(float) <= sizeof(S), "fp32 rows alias the slab");
-  __shared__ __attribute__((aligned(16))) float gtab[kGeluPolyLds];
   const int nres = kRows / K;
   const int r0 = blockIdx.x * nres;
   const int nr = min(nres, L - r0);
@@ -68,7 +67,6 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n0 = 32 * wave;
-  load_gelu_poly(gtab, threadIdx.x, blockDim.x);
   {
     // the tile's h_E rows, split: thread t loads float4 column t % 32 of rows t / 32 + 8 i, all loads
     // issued before the first store
@@ -123,8 +121,8 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
                                         : make_float4(0.F, 0.F, 0.F, 0.F);
         x = floatx4{a.x, a.y, a.z, a.w};
       }
-      const float4 o = row_t[rb] >= 0 ? make_float4(gelu_poly(x[0], gtab), gelu_poly(x[1], gtab),
-                                                    gelu_poly(x[2], gtab), gelu_poly(x[3], gtab))
+      const float4 o = row_t[rb] >= 0 ? make_float4(gelu_exp2(x[0]), gelu_exp2(x[1]),
+                                                    gelu_exp2(x[2]), gelu_exp2(x[3]))
                                       : make_float4(0.F, 0.F, 0.F, 0.F);
       put_split4(S, kRows, kLdS1, 16 * rb + r, c0, o);
     }
@@ -143,7 +141,7 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
         const float b = i == 0 ? bv.x : i == 1 ? bv.y : i == 2 ? bv.z : bv.w;
         float v = 0.0F;
 #pragma unroll
-        for (int rb = 0; rb < kRB; ++rb) v += row_t[rb] >= 0 ? gelu_poly(acc[rb][nt][i] + b, gtab) : 0.0F;
+        for (int rb = 0; rb < kRB; ++rb) v += row_t[rb] >= 0 ? gelu_exp2(acc[rb][nt][i] + b) : 0.0F;
         sv[i] = sum16(v);
       }
       if (r == 0) *reinterpret_cast<float4*>(msg_sum + (size_t)r0 * kH + c0) = make_float4(sv[0], sv[1], sv[2], sv[3]);
@@ -159,8 +157,8 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
     for (int rb = 0; rb < kRB; ++rb) {
       const floatx4 y = acc[rb][nt];
       *reinterpret_cast<float4*>(A + (16 * rb + r) * kLd + c0) =
-          row_t[rb] >= 0 ? make_float4(gelu_poly(y[0] + bv.x, gtab), gelu_poly(y[1] + bv.y, gtab),
-                                       gelu_poly(y[2] + bv.z, gtab), gelu_poly(y[3] + bv.w, gtab))
+          row_t[rb] >= 0 ? make_float4(gelu_exp2(y[0] + bv.x), gelu_exp2(y[1] + bv.y),
+                                       gelu_exp2(y[2] + bv.z), gelu_exp2(y[3] + bv.w))
                          : make_float4(0.F, 0.F, 0.F, 0.F);
     }
   }
@@ -180,8 +178,6 @@ __global__ __launch_bounds__(256, 3) void tf_node_kernel(ModelDev m, int layer, 
   __shared__ __attribute__((aligned(16))) float A[16 * kLd];
   __shared__ __attribute__((aligned(16))) float X[16 * kLd];
   __shared__ __attribute__((aligned(16))) float F[16 * kLdF];
-  __shared__ float tbl[17];
-  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
   const DecLayerDev& w = m.dec[layer];
   const int r0 = blockIdx.x * 16;
   const int wave = threadIdx.x >> 6;
@@ -221,7 +217,7 @@ __global__ __launch_bounds__(256, 3) void tf_node_kernel(ModelDev m, int layer, 
       for (int i = 0; i < 4; ++i) {
         const int row = 4 * (lane >> 4) + i;
         const int col = wave * 128 + nb * 16 + (lane & 15);
-        F[row * kLdF + col] = gelu(acc[nb][i] + w.bin[col], tbl);
+        F[row * kLdF + col] = gelu_exp2(acc[nb][i] + w.bin[col]);
       }
   }
   __syncthreads();

@@ -92,9 +92,9 @@ __device__ inline float gelu(float x, const float* tbl = kExpNegTable) {  // tbl
   return 0.5F * x * (1.0F + erfv);
 }
 
-// The same GELU formula for code held to a tolerance rather than to bit
-// identity (the 16-bit encoder's node kernel; the decode loop and the 16-bit
-// edge kernels use gelu_poly below): the exp table is read from LDS (tbl = 17
+// The same GELU formula held to a tolerance rather than to bit identity (the
+// yardstick of the device check beside gelu_poly and gelu_exp2 below, which
+// the kernels use): the exp table is read from LDS (tbl = 17
 // floats, kExpNegTable), 1/(1 + p v) is the hardware reciprocal (1 ulp) and
 // contraction is allowed. No v > 4 case is needed: there q is clamped to 16
 // and poly(t) exp(-16) < 2^-25, so mag rounds to exactly 1. The sign is copied
@@ -117,7 +117,7 @@ __device__ inline float gelu_fast(float x, const float* tbl) {
   return 0.5F * x * (1.0F + __builtin_copysignf(mag, x));
 }
 
-// The decode loop's GELU with the A&S term P(v) (erf = 1 - P) taken from a
+// The fp32 decode's FFN GELU with the A&S term P(v) (erf = 1 - P) taken from a
 // per-segment polynomial instead of the reciprocal, the Horner in t and the
 // exp Taylor polynomial (gelu_poly_gen.py fits the table to the reference
 // expression, within 7.4e-8 absolute; the segments keep the reference's exp
@@ -157,41 +157,39 @@ __device__ inline float gelu_poly(float x, const float* tab) {
   return 0.5F * x * (1.0F + __builtin_copysignf(mag, x));
 }
 
-__device__ inline floatx4 mfma16(float a, float b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+// GELU without a table, for the kernels that are held to a tolerance:
+//   gelu(x) = max(x, 0) - |x| E(|x|),   E(a) = P(a / sqrt(2)) / 2 = 2^p(a)
+// with P the A&S 7.1.26 term (erf = 1 - P) and p the degree-8 weighted minimax
+// fit of log2 E on [0, 5.6] (E within 2.6e-9 before rounding; p(0) = -1, so
+// gelu(x) -> x / 2). p has a negative leading coefficient and falls
+// monotonically past the range, so nothing is clamped; a NaN stays a NaN and
+// +-inf give NaN. Over all float inputs it is within 7.9e-8 |x| of the formula
+// in 64 bits (gelu_poly, which rounds 1 - P and 1 + erf as the reference does:
+// 4.6e-7 |x|). 8 FMAs, one exponential (four issue slots), a max and an FMA:
+// 14 VALU slots and no LDS read, against 20 and two 16-byte reads of gelu_poly,
+// which at 64 lanes take the LDS as long as the VALU and contend there with the
+// MFMA operands. The message rows, whose GELUs are 96 % of the decode's, run on
+// it: decode-bound designs 1.05x (L = 300 x 64) to 1.11x (4 x 256 x 256), split
+// bf16 at L = 4,000 1.11x, scoring 1.06x. The fp32 decode's FFN stays on
+// gelu_poly: a forced decode in 64 bits with each GELU exchanged in turn shows
+// that its roundings, and not the message rows', are the part of the
+// reference's own error (rms 5e-6 of log-prob at T = 0.2) that the fp32 decode
+// shares with it and that keeps the two within 1e-4 of each other.
+__device__ inline float gelu_exp2(float x) {
+  const float a = fabsf(x);
+  float p = __builtin_fmaf(a, -1.531581347e-06F, 2.223298907e-05F);
+  p = __builtin_fmaf(p, a, -9.656999464e-05F);
+  p = __builtin_fmaf(p, a, -3.706288408e-04F);
+  p = __builtin_fmaf(p, a, 7.382301148e-03F);
+  p = __builtin_fmaf(p, a, -5.271631479e-02F);
+  p = __builtin_fmaf(p, a, -4.591403008e-01F);
+  p = __builtin_fmaf(p, a, -1.151111841e+00F);
+  p = __builtin_fmaf(p, a, -1.0F);
+  return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.0F));
 }
 
-// One wave computes an (16 MB) x (16 NB) tile of A . W^T with fp32 MFMA.
-//   A : LDS, row-major with leading dimension lda (floats, multiple of 4).
-//   Wp: kpack16 weights of a layer with N output columns.
-//   n0: first output column of the wave's tile.
-// acc[mb][nb][i] holds D[row = 16 mb + 4 (lane / 16) + i][col = n0 + 16 nb + lane % 16].
-template <int MB, int NB>
-__device__ inline void mfma_tile(const float* __restrict__ A, int lda,
-                                 const float* __restrict__ Wp, int N, int n0, int kdim,
-                                 floatx4 (&acc)[MB][NB]) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15;
-  const int g = lane >> 4;
-  for (int kb = 0; kb < kdim / 16; ++kb) {
-    float4 a[MB];
-    float4 b[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-      b[nb] = *reinterpret_cast<const float4*>(Wp + ((size_t)kb * N + n0 + nb * 16 + r) * 16 + 4 * g);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      a[mb] = *reinterpret_cast<const float4*>(A + (mb * 16 + r) * lda + kb * 16 + 4 * g);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        acc[mb][nb] = mfma16(a[mb].x, b[nb].x, acc[mb][nb]);
-        acc[mb][nb] = mfma16(a[mb].y, b[nb].y, acc[mb][nb]);
-        acc[mb][nb] = mfma16(a[mb].z, b[nb].z, acc[mb][nb]);
-        acc[mb][nb] = mfma16(a[mb].w, b[nb].w, acc[mb][nb]);
-      }
-  }
+__device__ inline floatx4 mfma16(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 template <int MB, int NB>
@@ -200,6 +198,53 @@ __device__ inline void zero_acc(floatx4 (&acc)[MB][NB]) {
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = floatx4{0.F, 0.F, 0.F, 0.F};
+}
+
+// One wave computes an (16 MB) x (16 NB) tile of A . W^T with fp32 MFMA.
+//   A : LDS, row-major with leading dimension lda (floats, multiple of 4).
+//   Wp: kpack16 weights of a layer with N output columns.
+//   n0: first output column of the wave's tile.
+// acc[mb][nb][i] holds D[row = 16 mb + 4 (lane / 16) + i][col = n0 + 16 nb + lane % 16].
+// The sum runs in chains of 32 inputs that are then added (kdim a multiple of
+// 32): one chain of 128 rounded the decoder's E1 rows by 2.7e-6 rms of
+// log-prob at T = 0.2, most of the fp32 decode's own error, four chains by
+// 0.7e-6, and the shorter chains cost 32 adds per 32 inputs.
+template <int MB, int NB>
+__device__ inline void mfma_tile(const float* __restrict__ A, int lda,
+                                 const float* __restrict__ Wp, int N, int n0, int kdim,
+                                 floatx4 (&acc)[MB][NB]) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  zero_acc(acc);
+  for (int k0 = 0; k0 < kdim / 16; k0 += 2) {
+    floatx4 part[MB][NB];
+    zero_acc(part);
+#pragma unroll
+    for (int kb = k0; kb < k0 + 2; ++kb) {
+      float4 a[MB];
+      float4 b[NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        b[nb] = *reinterpret_cast<const float4*>(Wp + ((size_t)kb * N + n0 + nb * 16 + r) * 16 + 4 * g);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        a[mb] = *reinterpret_cast<const float4*>(A + (mb * 16 + r) * lda + kb * 16 + 4 * g);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          part[mb][nb] = mfma16(a[mb].x, b[nb].x, part[mb][nb]);
+          part[mb][nb] = mfma16(a[mb].y, b[nb].y, part[mb][nb]);
+          part[mb][nb] = mfma16(a[mb].z, b[nb].z, part[mb][nb]);
+          part[mb][nb] = mfma16(a[mb].w, b[nb].w, part[mb][nb]);
+        }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[mb][nb] += part[mb][nb];
+  }
 }
 
 // Writes an accumulator tile to LDS C (leading dimension ldc) at column n0.

@@ -7,8 +7,7 @@
 // fp16(v), lo = fp16((v - hi) * 2048)): hi.hi + (hi.lo + lo.hi) / 2048 in fp32
 // carries about 22 significant bits, so the encoder is fp32-accurate (not
 // the reference's rounding sequence, which encoder.hip reproduces). Features,
-// biases, GELU (gelu_poly in the edge kernels, gelu_fast in the node kernel),
-// LayerNorm (two-pass), residuals and the neighbour sum are fp32, and h_V, h_E
+// biases, GELU (gelu_exp2), LayerNorm (two-pass), residuals and the neighbour sum are fp32, and h_V, h_E
 // are stored in fp32. The kNN graph comes from the exact fp32 kernel.
 //
 // Edge products (the bulk of the work) run as workgroup tiles of 48 or 64 edge
@@ -57,14 +56,14 @@ static_assert(kEdgeIn % 32 == 0, "MFMA k-steps");
 // out[row][n0 + col] = GELU(acc + bias) (fp32) for the wave's 16 rows.
 template <int NT>
 __device__ inline void store_gelu(const floatx4 (&acc)[NT], const float* __restrict__ bias, int n0, float* out,
-                                  int ldo, const float* tbl) {
+                                  int ldo) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int col = n0 + 16 * nt + r;
     const float bv = bias[col];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[(4 * g + i) * ldo + col] = gelu_fast(acc[nt][i] + bv, tbl);
+    for (int i = 0; i < 4; ++i) out[(4 * g + i) * ldo + col] = gelu_exp2(acc[nt][i] + bv);
   }
 }
 
@@ -104,8 +103,7 @@ __device__ inline floatx4 edge_base(const float* __restrict__ P, size_t i, int j
 // GELU(acc + bias) of the wave's columns into the split slab (K = 128 operand
 // of the next product); no bias when bias is null.
 template <int RB>
-__device__ inline void tile_store_gelu(const floatx4 (&acc)[RB][2], const float* __restrict__ bias, _Float16* S,
-                                       const float* gtab) {
+__device__ inline void tile_store_gelu(const floatx4 (&acc)[RB][2], const float* __restrict__ bias, _Float16* S) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
@@ -113,8 +111,8 @@ __device__ inline void tile_store_gelu(const floatx4 (&acc)[RB][2], const float*
     const float4 bv = bias ? *reinterpret_cast<const float4*>(bias + c0) : make_float4(0.F, 0.F, 0.F, 0.F);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      const float4 v = make_float4(gelu_poly(acc[rb][nt][0] + bv.x, gtab), gelu_poly(acc[rb][nt][1] + bv.y, gtab),
-                                   gelu_poly(acc[rb][nt][2] + bv.z, gtab), gelu_poly(acc[rb][nt][3] + bv.w, gtab));
+      const float4 v = make_float4(gelu_exp2(acc[rb][nt][0] + bv.x), gelu_exp2(acc[rb][nt][1] + bv.y),
+                                   gelu_exp2(acc[rb][nt][2] + bv.z), gelu_exp2(acc[rb][nt][3] + bv.w));
       put_split4(S, 16 * RB, kLdS1, 16 * rb + r, c0, v);
     }
   }
@@ -335,11 +333,9 @@ __global__ __launch_bounds__(kTileThreads, 4) void edge_msg16_kernel(EncLayerDev
                                                                   float* __restrict__ gsum) {
   constexpr int RB = 3;
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * 16 * RB * kLdS1];
-  __shared__ __attribute__((aligned(16))) float gtab[kGeluPolyLds];
   const int res = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n0 = 32 * wave;
-  load_gelu_poly(gtab, threadIdx.x, kTileThreads);
   tile_rows<RB>(S, h_e, [&](int row) -> long long { return row < K ? (long long)res * K + row : -1; });
   // weight of slot 16 rb + r in the neighbour sum: mask_i mask_j / 30 for a valid slot
   float alpha[RB];
@@ -356,7 +352,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void edge_msg16_kernel(EncLayerDev
   // rows 128 .. 255 of W1 (packed k-blocks 16 .. 31) over e_ij, added to the h_i, h_j blocks and b1
   tile_gemm<RB, kH, 3>(S, kLdS1, w16.W1 + (size_t)16 * kH * 8, n0, (size_t)3 * kH * kH, acc, true);
   __syncthreads();  // every wave is done with e_ij
-  tile_store_gelu<RB>(acc, nullptr, S, gtab);
+  tile_store_gelu<RB>(acc, nullptr, S);
   __syncthreads();
   tile_gemm<RB, kH, 3>(S, kLdS1, w16.W2, n0, (size_t)kH * kH, acc);
 #pragma unroll
@@ -369,7 +365,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void edge_msg16_kernel(EncLayerDev
       const float b = i == 0 ? bv.x : i == 1 ? bv.y : i == 2 ? bv.z : bv.w;
       float v = 0.0F;
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) v += alpha[rb] * gelu_poly(acc[rb][nt][i] + b, gtab);
+      for (int rb = 0; rb < RB; ++rb) v += alpha[rb] * gelu_exp2(acc[rb][nt][i] + b);
       sv[i] = sum16(v);
     }
     if (r == 0) *reinterpret_cast<float4*>(gsum + (size_t)res * kH + c0) = make_float4(sv[0], sv[1], sv[2], sv[3]);
@@ -396,10 +392,8 @@ __global__ __launch_bounds__(256) void node16_kernel(EncLayerDev w, Enc16LayerDe
   __shared__ __attribute__((aligned(16))) float A[16 * kLdH];
   __shared__ __attribute__((aligned(16))) float F[16 * kLdF];
   __shared__ __attribute__((aligned(16))) float Pt[4][16 * kLdH];
-  __shared__ float tbl[17];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int r0 = blockIdx.x * 16;
-  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
   // the 16 rows of s into A (float4 column t % 32 of rows t / 32 and t / 32 + 8)
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
@@ -445,7 +439,7 @@ __global__ __launch_bounds__(256) void node16_kernel(EncLayerDev w, Enc16LayerDe
   __syncthreads();
   floatx4 acc[8];
   wave_gemm<8>(A, kLdH, w16.Win, kFF, kH * wave, kH, acc);
-  store_gelu<8>(acc, w.bin, kH * wave, F, kLdF, tbl);
+  store_gelu<8>(acc, w.bin, kH * wave, F, kLdF);
   __syncthreads();
   // inputs [128 w, 128 w + 128) of W_out: its packed rows 16 w .. 16 w + 15
   wave_gemm<8>(F + kH * wave, kLdF, w16.Wout + (size_t)wave * 16 * kH * 8, kH, 0, kH, acc, (size_t)kFF * kH);
@@ -503,10 +497,8 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_update16_kernel(EncLayer
   constexpr int RB = 4;
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * 16 * RB * kLdS1];
   __shared__ float stat[4][16 * RB];
-  __shared__ __attribute__((aligned(16))) float gtab[kGeluPolyLds];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n0 = 32 * wave;
-  load_gelu_poly(gtab, threadIdx.x, kTileThreads);
   const long long S_ = (long long)L * K;
   const long long base = (long long)blockIdx.x * 16 * RB;
   tile_rows<RB>(S, h_e, [&](int row) -> long long { return base + row < S_ ? base + row : -1; });
@@ -523,11 +515,11 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_update16_kernel(EncLayer
   // rows 128 .. 255 of W11 (packed k-blocks 16 .. 31) over e_ij, added to the h_i, h_j blocks and b11
   tile_gemm<RB, kH, 3>(S, kLdS1, w16.W11 + (size_t)16 * kH * 8, n0, (size_t)3 * kH * kH, acc, true);
   __syncthreads();
-  tile_store_gelu<RB>(acc, nullptr, S, gtab);
+  tile_store_gelu<RB>(acc, nullptr, S);
   __syncthreads();
   tile_gemm<RB, kH, 3>(S, kLdS1, w16.W12, n0, (size_t)kH * kH, acc);
   __syncthreads();
-  tile_store_gelu<RB>(acc, w.b12, S, gtab);
+  tile_store_gelu<RB>(acc, w.b12, S);
   // x = (e + b13) + W13 g: the residual rows start the last product's accumulators
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {

@@ -175,6 +175,65 @@ extern "C" int hkbs_check_device_gelu(unsigned long long* counts_out, unsigned i
 
 namespace {
 
+// gelu_exp2 and gelu_poly against the A&S formula in 64 bits, on every float input with |x| <= 1e4:
+// worst[0], worst[1] = the largest |got - formula| / |x| (float bits) of the two; bad = NaN inputs whose
+// gelu_exp2 is not a NaN, plus larger finite inputs where it is not max(x, 0) to 1e-7 |x|.
+__global__ void gelu_exp2_kernel(unsigned int* worst, unsigned long long* bad) {
+  __shared__ __attribute__((aligned(16))) float gtab[hkbs::kGeluPolyLds];
+  hkbs::load_gelu_poly(gtab, threadIdx.x, blockDim.x);
+  __syncthreads();
+  float w0 = 0.0F, w1 = 0.0F;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t bits = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; bits < (1ull << 32); bits += stride) {
+    const float x = __uint_as_float(static_cast<unsigned int>(bits));
+    const float got = hkbs::gelu_exp2(x);
+    if (x != x) {
+      if (got == got) atomicAdd(bad, 1ull);
+      continue;
+    }
+    if (!isfinite(x) || x == 0.0F) continue;
+    if (fabsf(x) > 1.0e4F) {
+      if (!(fabsf(got - fmaxf(x, 0.0F)) <= 1.0e-7F * fabsf(x))) atomicAdd(bad, 1ull);
+      continue;
+    }
+    const double a = fabs((double)x), v = a * 0.70710678118654752440, t = 1.0 / (1.0 + 0.3275911 * v);
+    const double P =
+        (((((1.061405429 * t - 1.453152027) * t) + 1.421413741) * t - 0.284496736) * t + 0.254829592) * t * exp(-v * v);
+    const double ref = (x > 0.0F ? a : 0.0) - 0.5 * a * P;
+    // results below the smallest normal float are flushed: an absolute allowance of 2^-126
+    const double d0 = fmax(0.0, fabs((double)got - ref) - 1.2e-38) / a;
+    const double d1 = fmax(0.0, fabs((double)hkbs::gelu_poly(x, gtab) - ref) - 1.2e-38) / a;
+    w0 = fmaxf(w0, (float)d0);
+    w1 = fmaxf(w1, (float)d1);
+  }
+  atomicMax(&worst[0], __float_as_uint(w0));
+  atomicMax(&worst[1], __float_as_uint(w1));
+}
+
+}  // namespace
+
+// worst_out[2] and bad_out as in gelu_exp2_kernel. Returns the HIP status of the run.
+extern "C" int hkbs_check_device_gelu_exp2(unsigned int* worst_out, unsigned long long* bad_out) {
+  unsigned int* worst = nullptr;
+  unsigned long long* bad = nullptr;
+  hipError_t e = hipMalloc(&worst, 2 * sizeof(unsigned int));
+  if (e == hipSuccess) e = hipMalloc(&bad, sizeof(unsigned long long));
+  if (e == hipSuccess) e = hipMemset(worst, 0, 2 * sizeof(unsigned int));
+  if (e == hipSuccess) e = hipMemset(bad, 0, sizeof(unsigned long long));
+  if (e == hipSuccess) {
+    gelu_exp2_kernel<<<8192, 256>>>(worst, bad);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipMemcpy(worst_out, worst, 2 * sizeof(unsigned int), hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(bad_out, bad, sizeof(unsigned long long), hipMemcpyDeviceToHost);
+  if (worst) (void)hipFree(worst);
+  if (bad) (void)hipFree(bad);
+  return static_cast<int>(e);
+}
+
+namespace {
+
 // rbf_chunk_fma (16-bit encoder) against rbf_chunk (the reference's operation
 // order) for n atom-pair offsets: offset i has length 30 i / n Angstrom along
 // a direction that turns with i. out[0] = the largest |fma - ref| / ref over
