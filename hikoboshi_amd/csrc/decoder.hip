@@ -239,7 +239,7 @@ __device__ inline void put_split16(uint16_t* hi, int lo_at, float v) {
     const float c = __builtin_amdgcn_fmed3f(v, -65504.0F, 65504.0F);
     const _Float16 h = static_cast<_Float16>(c);
     hi[0] = __builtin_bit_cast(uint16_t, h);
-    hi[lo_at] = __builtin_bit_cast(uint16_t, static_cast<_Float16>((c - static_cast<float>(h)) * 2048.0F));
+    hi[lo_at] = __builtin_bit_cast(uint16_t, split_lo(c, h));
   }
 }
 
@@ -884,7 +884,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
                     for (int e = 0; e < 4; ++e) {
                       const float cl = __builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F);
                       hv[e] = static_cast<_Float16>(cl);
-                      lv[e] = static_cast<_Float16>((vv[e] - static_cast<float>(hv[e])) * 2048.0F);
+                      lv[e] = split_lo(vv[e], hv[e]);
                     }
                     *reinterpret_cast<half4*>(gh) = hv;
                     *reinterpret_cast<half4*>(gl) = lv;
@@ -1453,7 +1453,7 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
       for (int e = 0; e < 4; ++e) {
         const float cl = __builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F);
         hv[e] = static_cast<_Float16>(cl);
-        lv[e] = static_cast<_Float16>((vv[e] - static_cast<float>(hv[e])) * 2048.0F);
+        lv[e] = split_lo(vv[e], hv[e]);
       }
       *reinterpret_cast<half4*>(G16 + row * kLdH + c) = hv;
       *reinterpret_cast<half4*>(G16 + (kKmax + row) * kLdH + c) = lv;

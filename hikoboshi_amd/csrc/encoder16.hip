@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_embed16_kernel(ModelDev 
           const float f = out[8 * q + e];
           const _Float16 hi = static_cast<_Float16>(__builtin_amdgcn_fmed3f(f, -65504.0F, 65504.0F));
           h[e] = hi;
-          l[e] = static_cast<_Float16>((f - static_cast<float>(hi)) * 2048.0F);
+          l[e] = split_lo(f, hi);
         }
         *reinterpret_cast<f16x8*>(S + row * kLdE + 16 * (c - c0) + 8 * q) = h;
         *reinterpret_cast<f16x8*>(S + (R + row) * kLdE + 16 * (c - c0) + 8 * q) = l;

@@ -72,7 +72,7 @@ __device__ inline void wave_gemm(const float* A, int lda, const uint16_t* __rest
     for (int e = 0; e < 8; ++e) {
       const float v = __builtin_amdgcn_fmed3f(av[e], -65504.0F, 65504.0F);
       ah[e] = static_cast<_Float16>(v);
-      al[e] = static_cast<_Float16>((av[e] - static_cast<float>(ah[e])) * 2048.0F);
+      al[e] = split_lo(av[e], ah[e]);
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -111,7 +111,7 @@ __device__ inline void put_split4(_Float16* S, int rows, int ld, int row, int co
   for (int e = 0; e < 4; ++e) {
     const _Float16 hi = static_cast<_Float16>(__builtin_amdgcn_fmed3f(f[e], -65504.0F, 65504.0F));
     h[e] = hi;
-    l[e] = static_cast<_Float16>((f[e] - static_cast<float>(hi)) * 2048.0F);
+    l[e] = split_lo(f[e], hi);
   }
   *reinterpret_cast<f16x4*>(S + row * ld + col) = h;
   *reinterpret_cast<f16x4*>(S + (rows + row) * ld + col) = l;
