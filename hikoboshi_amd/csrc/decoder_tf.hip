@@ -11,7 +11,7 @@
 // kernel, every edge is used once per layer), R^l_j = W1d h^l_j +
 // W1c W_s[tok_j] and Q^l_j = W1d h^0_j; and sum_k (W3 g_k + b3) = W3 sum_k g_k + K b3.
 // Per layer:
-//   tf_edge_kernel  tiles of whole residues (<= 48 edge rows): W1b and W2 on the
+//   tf_edge_kernel  one residue (<= 48 edge rows) per workgroup: W1b and W2 on the
 //                   fp16 MFMA with split operands (hi + lo / 2048 for weights and
 //                   rows, about 22 significant bits), GELU, neighbour sum (all K
 //                   slots, no attention mask).
@@ -28,7 +28,6 @@
 namespace hkbs {
 namespace {
 
-constexpr int kRows = 48;
 constexpr int kLd = kH + 4;
 constexpr int kLdF = kFF + 4;
 
@@ -43,32 +42,26 @@ __global__ void tf_init_kernel(ModelDev m, const float* __restrict__ Q, const in
   NB[r * 256 + kH + c] = Q[r * kH + c] + m.dec[0].T[tokens[r] * kH + c];
 }
 
-// One tile of kRows edge rows per workgroup: the K slots of kRows / K
-// consecutive residues (one residue when K = 48), their h_E rows split into
-// fp16 halves in LDS (hi [kRows][kLdS1] then lo, the layout of tile_gemm).
-constexpr int kRB = kRows / 16;
-static_assert(kRows % 16 == 0 && kRows >= kKmax, "a tile holds whole residues");
-
+// One residue per workgroup: its K <= 16 RB slots (rows past its own neighbour
+// count are zero) as a tile of 16 RB edge rows, split into fp16 halves in LDS
+// (hi [16 RB][kLdS1] then lo, the layout of tile_gemm). Rows do not depend on
+// each other before the sum over the residue's slots, so the result is the same
+// whatever K the batch was laid out with.
+template <int kRB>
 __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const float* __restrict__ h_e,
                                                       const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
                                                       const float* __restrict__ mask, const float* __restrict__ NB,
                                                       const float* __restrict__ Ql, int L, int K,
                                                       float* __restrict__ msg_sum) {
-  // The split h_E slab; once the W2 product has read it, the same bytes hold
-  // the fp32 message rows [kRows][kLd] for the neighbour sums (K < 48).
-  __shared__ __attribute__((aligned(16))) _Float16 S[2 * kRows * kLdS1];
-  float* A = reinterpret_cast<float*>(S);
-  static_assert(kRows * kLd * sizeof(float) <= sizeof(S), "fp32 rows alias the slab");
-  const int nres = kRows / K;
-  const int r0 = blockIdx.x * nres;
-  const int nr = min(nres, L - r0);
-  const int n_rows = nr * K;
-  const size_t slot0 = (size_t)r0 * K;
+  constexpr int kRows = 16 * kRB;
+  __shared__ __attribute__((aligned(16))) _Float16 S[2 * kRows * kLdS1];  // the split h_E rows, then the GELU rows
+  const int t = blockIdx.x;
+  const size_t slot0 = (size_t)t * K;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n0 = 32 * wave;
   {
-    // the tile's h_E rows, split: thread t loads float4 column t % 32 of rows t / 32 + 8 i, all loads
+    // the residue's h_E rows, split: thread i loads float4 column i % 32 of rows i / 32 + 8 n, all loads
     // issued before the first store
     constexpr int N = kRows * (kH / 4) / 256;
     const int col = 4 * (threadIdx.x & 31), row0 = threadIdx.x >> 5;
@@ -76,31 +69,27 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int row = row0 + 8 * i;
-      v[i] = row < n_rows ? *reinterpret_cast<const float4*>(h_e + (slot0 + row) * kH + col)
-                          : make_float4(0.F, 0.F, 0.F, 0.F);
+      v[i] = row < K ? *reinterpret_cast<const float4*>(h_e + (slot0 + row) * kH + col) : make_float4(0.F, 0.F, 0.F, 0.F);
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) put_split4(S, kRows, kLdS1, row0 + 8 * i, col, v[i]);
   }
-  // Row 16 rb + r: its residue t and whether the slot adds a context (j a residue, t not masked). Then
-  // x = A_t + (bw ? R_j : Q_j) + E1 with E1 = W1b h_E for a slot that adds one, else x = A_t: the
+  // Row 16 rb + r: whether it is a slot of the residue, and whether the slot adds a context (j a residue, t not
+  // masked). Then x = A_t + (bw ? R_j : Q_j) + E1 with E1 = W1b h_E for a slot that adds one, else x = A_t: the
   // accumulators start at A_t + (R_j or Q_j) and the W1b product adds E1.
-  int row_t[kRB];
-  bool adds[kRB];
+  bool valid[kRB], adds[kRB];
   floatx4 acc[kRB][2];
 #pragma unroll
   for (int rb = 0; rb < kRB; ++rb) {
     const int row = 16 * rb + r;
-    const bool valid = row < n_rows;
-    const int t = r0 + (valid ? row / K : 0);
-    const int j = valid ? idx[slot0 + row] : -1;
-    adds[rb] = valid && j >= 0 && j < L && mask[t] != 0.0F;
+    const int j = row < K ? idx[slot0 + row] : kNoSlot;
+    valid[rb] = j != kNoSlot;
+    adds[rb] = j >= 0 && j < L && mask[t] != 0.0F;
     const bool bw = adds[rb] && pos[j] < pos[t];
-    row_t[rb] = valid ? t : -1;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       const int c0 = n0 + 16 * nt + 4 * g;
-      const float4 x = valid ? *reinterpret_cast<const float4*>(NB + (size_t)t * 256 + c0) : make_float4(0.F, 0.F, 0.F, 0.F);
+      const float4 x = *reinterpret_cast<const float4*>(NB + (size_t)t * 256 + c0);
       const float4 e = !adds[rb] ? make_float4(0.F, 0.F, 0.F, 0.F)
                                  : *reinterpret_cast<const float4*>(bw ? NB + (size_t)j * 256 + kH + c0
                                                                        : Ql + (size_t)j * kH + c0);
@@ -116,70 +105,54 @@ __global__ __launch_bounds__(256, 4) void tf_edge_kernel(DecLayerDev w, const fl
     for (int nt = 0; nt < 2; ++nt) {
       const int c0 = n0 + 16 * nt + 4 * g;
       floatx4 x = acc[rb][nt];
-      if (!adds[rb]) {  // A_t alone (zero for a row past the tile's residues)
-        const float4 a = row_t[rb] >= 0 ? *reinterpret_cast<const float4*>(NB + (size_t)row_t[rb] * 256 + c0)
-                                        : make_float4(0.F, 0.F, 0.F, 0.F);
+      if (!adds[rb]) {  // A_t alone
+        const float4 a = *reinterpret_cast<const float4*>(NB + (size_t)t * 256 + c0);
         x = floatx4{a.x, a.y, a.z, a.w};
       }
-      const float4 o = row_t[rb] >= 0 ? make_float4(gelu_exp2(x[0]), gelu_exp2(x[1]),
-                                                    gelu_exp2(x[2]), gelu_exp2(x[3]))
-                                      : make_float4(0.F, 0.F, 0.F, 0.F);
+      const float4 o = valid[rb] ? make_float4(gelu_exp2(x[0]), gelu_exp2(x[1]), gelu_exp2(x[2]), gelu_exp2(x[3]))
+                                 : make_float4(0.F, 0.F, 0.F, 0.F);
       put_split4(S, kRows, kLdS1, 16 * rb + r, c0, o);
     }
   }
   __syncthreads();
   tile_gemm<kRB, kH, 3>(S, kLdS1, reinterpret_cast<const uint16_t*>(w.W2h), n0, (size_t)kH * kH, acc);
-  // g = GELU(W2 x + b2) per valid row; msg_sum[t] = the sum over the residue's K slots
-  if (nres == 1) {
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const int c0 = n0 + 16 * nt + 4 * g;
-      const float4 bv = *reinterpret_cast<const float4*>(w.b2 + c0);
-      float sv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float b = i == 0 ? bv.x : i == 1 ? bv.y : i == 2 ? bv.z : bv.w;
-        float v = 0.0F;
-#pragma unroll
-        for (int rb = 0; rb < kRB; ++rb) v += row_t[rb] >= 0 ? gelu_exp2(acc[rb][nt][i] + b) : 0.0F;
-        sv[i] = sum16(v);
-      }
-      if (r == 0) *reinterpret_cast<float4*>(msg_sum + (size_t)r0 * kH + c0) = make_float4(sv[0], sv[1], sv[2], sv[3]);
-    }
-    return;
-  }
-  __syncthreads();  // the slab is consumed; A reuses its bytes
+  // g = GELU(W2 x + b2) per slot; msg_sum[t] = the sum over the residue's slots
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
     const int c0 = n0 + 16 * nt + 4 * g;
     const float4 bv = *reinterpret_cast<const float4*>(w.b2 + c0);
+    float sv[4];
 #pragma unroll
-    for (int rb = 0; rb < kRB; ++rb) {
-      const floatx4 y = acc[rb][nt];
-      *reinterpret_cast<float4*>(A + (16 * rb + r) * kLd + c0) =
-          row_t[rb] >= 0 ? make_float4(gelu_exp2(y[0] + bv.x), gelu_exp2(y[1] + bv.y),
-                                       gelu_exp2(y[2] + bv.z), gelu_exp2(y[3] + bv.w))
-                         : make_float4(0.F, 0.F, 0.F, 0.F);
+    for (int i = 0; i < 4; ++i) {
+      const float b = i == 0 ? bv.x : i == 1 ? bv.y : i == 2 ? bv.z : bv.w;
+      float v = 0.0F;
+#pragma unroll
+      for (int rb = 0; rb < kRB; ++rb) v += valid[rb] ? gelu_exp2(acc[rb][nt][i] + b) : 0.0F;
+      sv[i] = sum16(v);
     }
-  }
-  __syncthreads();
-  for (int task = threadIdx.x; task < nr * kH; task += blockDim.x) {
-    const int lr = task / kH, c = task % kH;
-    float s = 0.0F;
-    for (int k = 0; k < K; ++k) s += A[(lr * K + k) * kLd + c];
-    msg_sum[(size_t)(r0 + lr) * kH + c] = s;
+    if (r == 0) *reinterpret_cast<float4*>(msg_sum + (size_t)t * kH + c0) = make_float4(sv[0], sv[1], sv[2], sv[3]);
   }
 }
 
 __global__ __launch_bounds__(256, 3) void tf_node_kernel(ModelDev m, int layer, const float* __restrict__ msg_sum,
                                                       const float* __restrict__ mask, const int32_t* __restrict__ tokens,
-                                                      int L, int K, float* __restrict__ h, float* __restrict__ NB,
-                                                      float* __restrict__ log_probs) {
+                                                      int L, int K, const int32_t* __restrict__ seg,
+                                                      const int64_t* __restrict__ offsets, float* __restrict__ h,
+                                                      float* __restrict__ NB, float* __restrict__ log_probs) {
   __shared__ __attribute__((aligned(16))) float A[16 * kLd];
   __shared__ __attribute__((aligned(16))) float X[16 * kLd];
   __shared__ __attribute__((aligned(16))) float F[16 * kLdF];
+  __shared__ float slots[16];  // neighbour slots of each row's residue: K, or its protein's length where that is less
   const DecLayerDev& w = m.dec[layer];
   const int r0 = blockIdx.x * 16;
+  if (threadIdx.x < 16) {
+    int n = K;
+    if (seg && r0 + (int)threadIdx.x < L) {
+      const int p = seg[r0 + threadIdx.x];
+      n = min(K, static_cast<int>(offsets[p + 1] - offsets[p]));
+    }
+    slots[threadIdx.x] = static_cast<float>(n);
+  }
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
 
@@ -201,7 +174,7 @@ __global__ __launch_bounds__(256, 3) void tf_node_kernel(ModelDev m, int layer, 
         const int col = wave * 32 + nb * 16 + (lane & 15);
         float v = 0.0F;
         if (r0 + row < L)
-          v = h[(size_t)(r0 + row) * kH + col] + (acc[nb][i] + static_cast<float>(K) * w.b3[col]) * (1.0F / 30.0F);
+          v = h[(size_t)(r0 + row) * kH + col] + (acc[nb][i] + slots[row] * w.b3[col]) * (1.0F / 30.0F);
         X[row * kLd + col] = v;
       }
   }
@@ -293,13 +266,14 @@ hipError_t launch_teacher_forced(const ModelDev& m, const TfArgs& a, hipStream_t
   const int L = a.L, K = a.K;
   if (L <= 0) return hipSuccess;
   tf_init_kernel<<<(unsigned)(((size_t)L * kH + 255) / 256), 256, 0, stream>>>(m, a.Q, a.tokens, L, a.NB);
-  const int nres = kRows / K;
-  const unsigned edge_tiles = (unsigned)((L + nres - 1) / nres);
+  if (K < 1 || K > kKmax) return hipErrorInvalidValue;
   const unsigned node_tiles = (unsigned)((L + 15) / 16);
   for (int l = 0; l < kLayers; ++l) {
-    tf_edge_kernel<<<edge_tiles, 256, 0, stream>>>(m.dec[l], a.h_e, a.idx, a.pos, a.mask, a.NB,
-                                                   a.Q + (size_t)l * L * kH, L, K, a.msg_sum);
-    tf_node_kernel<<<node_tiles, 256, 0, stream>>>(m, l, a.msg_sum, a.mask, a.tokens, L, K, a.h, a.NB, a.log_probs);
+    // as few blocks of 16 rows as hold the K slots (short proteins)
+    auto* edge = K <= 16 ? tf_edge_kernel<1> : K <= 32 ? tf_edge_kernel<2> : tf_edge_kernel<3>;
+    edge<<<(unsigned)L, 256, 0, stream>>>(m.dec[l], a.h_e, a.idx, a.pos, a.mask, a.NB, a.Q + (size_t)l * L * kH, L, K,
+                                          a.msg_sum);
+    tf_node_kernel<<<node_tiles, 256, 0, stream>>>(m, l, a.msg_sum, a.mask, a.tokens, L, K, a.seg, a.offsets, a.h, a.NB, a.log_probs);
   }
   return hipGetLastError();
 }

@@ -29,7 +29,7 @@
 //   edge_embed16   64 edge slots per workgroup (4 waves): 416 features ->
 //                  W_edge -> LN -> W_e -> h_E.
 //   per layer:
-//   edge_msg16     one residue per workgroup (48 slots, 4 waves): W1 e_ij +
+//   edge_msg16     one residue per workgroup (up to 48 slots, 4 waves): W1 e_ij +
 //                  P, GELU, W2, GELU -> the sum over the residue's slots
 //                  weighted by mask_i mask_j / 30, and the sum of the weights.
 //   node16         16 residues per workgroup (4 waves): upd = W3 sum + (sum of
@@ -49,7 +49,7 @@ namespace {
 
 constexpr int kLdF = kFF + 4;      // floats per row of the FFN hidden layer
 constexpr int kLdH = kH + 4;       // floats per row of a 128-wide activation
-static_assert(kKmax == 48, "edge_msg16 covers a residue's slots with 3 waves of 16 rows");
+static_assert(kKmax == 48, "edge_msg16 covers a residue's slots with up to 3 blocks of 16 rows");
 static_assert(kEdgeIn % 32 == 0, "MFMA k-steps");
 
 
@@ -319,19 +319,19 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_embed16_kernel(ModelDev 
   }
 }
 
-// One residue per workgroup: its 48 slots as one tile of 3 row blocks. The
+// One residue per workgroup: its K <= 16 RB slots as one tile of RB row blocks. The
 // message of slot k is m_k = W3 g_k + b3 with g_k = GELU(W2 GELU(W1 x_k + b1) +
 // b2), and upd_i = sum_k alpha_k m_k = W3 (sum_k alpha_k g_k) + (sum_k alpha_k)
 // b3, so this kernel stops at s_i = sum_k alpha_k g_k and a_i = sum_k alpha_k
 // (gsum[i][0 .. 127] and gsum[128 L + i]); node16 applies W3 to 16 residues
 // at a time.
+template <int RB>
 __global__ __launch_bounds__(kTileThreads, 4) void edge_msg16_kernel(EncLayerDev w, Enc16LayerDev w16,
                                                                   const float* __restrict__ h_e,
                                                                   const int32_t* __restrict__ idx,
                                                                   const float* __restrict__ mask,
                                                                   const float* __restrict__ prefix, int L, int K,
                                                                   float* __restrict__ gsum) {
-  constexpr int RB = 3;
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * 16 * RB * kLdS1];
   const int res = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -572,8 +572,9 @@ hipError_t launch_encoder16(const ModelDev& m, const float* coords, const uint8_
   for (int l = 0; l < kLayers; ++l) {
     const Enc16LayerDev& w16 = m.enc16.layer[l];
     const uint16_t* W1_next = l + 1 < kLayers ? m.enc16.layer[l + 1].W1 : nullptr;
-    edge_msg16_kernel<<<(unsigned)L, kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, mask, ws.prefix, L, K,
-                                                                 gsum);
+    // as few blocks of 16 rows as hold the K slots (short proteins)
+    auto* msg = K <= 16 ? edge_msg16_kernel<1> : K <= 32 ? edge_msg16_kernel<2> : edge_msg16_kernel<3>;
+    msg<<<(unsigned)L, kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, mask, ws.prefix, L, K, gsum);
     node16_kernel<<<(unsigned)((L + 15) / 16), 256, 0, stream>>>(m.enc[l], w16, gsum, mask, L, h_v, W1_next,
                                                                 ws.prefix);
     edge_update16_kernel<<<tiles64, kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, ws.prefix, L, K);

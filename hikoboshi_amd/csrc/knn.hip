@@ -83,7 +83,9 @@ __global__ void prep_ca_kernel(const float* __restrict__ coords, const uint8_t* 
 }
 
 // Rows of a ragged batch (seg != null) only see the residues of their own
-// protein, [offsets[seg[q]], offsets[seg[q] + 1]); indices stay global.
+// protein, [offsets[seg[q]], offsets[seg[q] + 1]); indices stay global. A
+// protein of fewer than K residues has that many neighbour slots; its rows'
+// remaining slots hold kNoSlot.
 __global__ __launch_bounds__(256) void knn_kernel(const float4* __restrict__ ca, int L, int K,
                                                   const int32_t* __restrict__ seg, const int64_t* __restrict__ offsets,
                                                   int32_t* __restrict__ idx, float* __restrict__ d2) {
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(256) void knn_kernel(const float4* __restrict__ ca,
   if (lane < K) {
     const size_t o = (size_t)q * K + lane;
     if (best == kNone) {
-      idx[o] = -1;
+      idx[o] = lane < hi - lo ? -1 : kNoSlot;
       d2[o] = row_max;
     } else {
       idx[o] = static_cast<int32_t>(best & 0xffffffffu);

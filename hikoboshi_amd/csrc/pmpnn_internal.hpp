@@ -11,6 +11,7 @@ namespace hkbs {
 constexpr int kH = 128;        // hidden width
 constexpr int kV = 21;         // vocabulary
 constexpr int kKmax = 48;      // neighbours
+constexpr int kNoSlot = -2;    // idx of a slot past its protein's own neighbour count (ragged batches); -1: empty slot
 constexpr int kRbf = 16;       // RBF centres
 constexpr int kPairs = 25;     // atom pairs
 constexpr int kPos = 16;       // positional features
@@ -263,6 +264,8 @@ struct TfArgs {
   float* msg_sum;         // [L][128] workspace
   float* log_probs;       // [L][21] output
   int L, K;
+  const int32_t* seg;     // ragged batch: protein of each row, and the proteins' row offsets (null: one protein)
+  const int64_t* offsets;
 };
 hipError_t launch_teacher_forced(const ModelDev& m, const TfArgs& a, hipStream_t stream);
 

@@ -1,0 +1,28 @@
+"""Ragged scoring of short proteins: chunks laid out with more slots than a protein has neighbours."""
+import numpy as np
+import pytest
+
+from hikoboshi_amd import backbone
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens", [[1, 2, 15, 16, 17], [47, 48, 49], [33, 16, 60, 31, 32, 1, 48], [5] * 3 + [90] + [20] * 4])
+def test_short_proteins_share_a_chunk(gpu_ctx, oracle, lens):
+    """Proteins around the row-block and neighbour-count edges in one call: bit-identical to scoring each alone
+    (its own K), and within 1e-4 of the oracle; one residue without backbone atoms in every protein longer than 4."""
+    parts = [backbone.single_chain(n, 30 + i) for i, n in enumerate(lens)]
+    for bb in parts:
+        if bb.L > 4:
+            bb.atom_sources[3, 1] = 0
+    tok = [backbone.native_tokens(n, np.random.default_rng(n)) for n in lens]
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    print("score", lens, flush=True)
+    lp, sc = gpu_ctx.score_batch(np.concatenate([b.coords for b in parts]),
+                                 np.concatenate([b.atom_sources for b in parts]), np.concatenate(tok), off)
+    for i, bb in enumerate(parts):
+        one_lp, one_sc = gpu_ctx.score(bb.coords, bb.atom_sources, tok[i])
+        np.testing.assert_array_equal(lp[off[i]:off[i + 1]], one_lp)
+        assert sc[i] == np.float32(one_sc)
+        olp, oscore = oracle.teacher_forced(bb, tok[i])
+        assert np.abs(one_lp - olp).max() <= 1e-4
