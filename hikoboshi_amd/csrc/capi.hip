@@ -949,12 +949,13 @@ hkbs_status adopt_caller_stream(hkbs_pmpnn* ctx, void* stream, bool* capturing) 
   return HKBS_OK;
 }
 
-// Shared implementation of the device design path. All pointers device.
+// Shared implementation of the device design path. All pointers device. keeps = false: the caller knows that every
+// order's first step samples a token, so that there is no kept prefix to look for.
 hkbs_status design_on_device(hkbs_pmpnn* ctx, const float* coords, const uint8_t* src, const int32_t* resid,
                              const int32_t* chain, const float* chain_mask, const int32_t* true_tokens, int L, int B,
                              const int32_t* orders, int shared, const uint64_t* seeds, float temperature, int greedy,
                              int32_t* tokens, float* log_probs, float* scores, DeviceArena& ar, float* chosen,
-                             bool l0table) {
+                             bool l0table, bool keeps = true) {
   // The decode runs as an ordinary launch whose grid is resident at once, with
   // bounded team barriers; a cooperative launch is not offered.
   if (const char* mode = std::getenv("HKBS_DECODE_LAUNCH"); mode && std::strcmp(mode, "cooperative") == 0)
@@ -1025,6 +1026,11 @@ hkbs_status design_on_device(hkbs_pmpnn* ctx, const float* coords, const uint8_t
     a.Rh = reinterpret_cast<_Float16*>(R);
     a.E1 = nullptr;
   }
+  // Words for the kept prefixes lie in the kNN distances, which the path does not use. HKBS_DECODE_PREFIX=off leaves
+  // the prefix to the pass loop.
+  const char* pre = std::getenv("HKBS_DECODE_PREFIX");
+  if (chain_mask && keeps && K >= kPrefixMinK && 2 * nq <= S && !(pre && std::strcmp(pre, "off") == 0))
+    a.prefix = reinterpret_cast<const int32_t*>(e.d2);
   const int team = decode_team_size(a.precision, B, 8);
   a.max_members = decode_group(a.precision, team) * team;
   a.pass_granule = team;
@@ -1041,7 +1047,8 @@ hkbs_status design_on_device(hkbs_pmpnn* ctx, const float* coords, const uint8_t
   HK_CHECK(launch_featurise_encode(ctx, coords, src, resid, chain, L, K, e), "encoder launch failed");
   HK_CHECK(hipStreamWaitEvent(ctx->side, ctx->fork, 0), "stream wait failed");
   HK_CHECK(launch_positions(orders, L, shared ? 1 : B, shared, pos, ctx->side), "position kernel failed");
-  if (l0base) HK_CHECK(launch_l0_rows(e.idx, pos, L, K, l0base, ctx->side), "layer-0 table rows failed");
+  HK_CHECK(launch_prefix_steps(a, ctx->side), "prefix kernel failed");
+  if (l0base) HK_CHECK(launch_l0_rows(e.idx, pos, a.prefix, L, K, l0base, ctx->side), "layer-0 table rows failed");
   HK_CHECK(hipEventRecord(ctx->rows, ctx->side), "event record failed");
   HK_CHECK(launch_decode_schedule(a, ctx->side), "decode schedule launch failed");
   HK_CHECK(hipEventRecord(ctx->join, ctx->side), "event record failed");
@@ -1051,12 +1058,24 @@ hkbs_status design_on_device(hkbs_pmpnn* ctx, const float* coords, const uint8_t
            "decoder precompute failed");
   HK_CHECK(launch_zero(reinterpret_cast<float*>(sync), (size_t)B + 1, ctx->stream), "workspace clear failed");
   // The table needs the positions and its row offsets; it is built while the
-  // schedule (a few workgroups on the side stream) may still run.
+  // schedule (a few workgroups on the side stream) may still run, unless a kept
+  // prefix, which reads its step records, comes before it.
+  const auto table = [&]() -> hkbs_status {
+    if (l0tab)
+      HK_CHECK(launch_layer0_table(ctx->model, E1, Q, e.idx, pos, l0base, a.prefix, L, K, l0tab, ctx->stream),
+               "layer-0 table failed");
+    return HKBS_OK;
+  };
+  hkbs_status st = HKBS_OK;
   HK_CHECK(hipStreamWaitEvent(ctx->stream, ctx->rows, 0), "stream wait failed");
-  if (l0tab)
-    HK_CHECK(launch_layer0_table(ctx->model, E1, Q, e.idx, pos, l0base, L, K, l0tab, ctx->stream), "layer-0 table failed");
+  if (!a.prefix && (st = table()) != HKBS_OK) return st;
   HK_CHECK(hipStreamWaitEvent(ctx->stream, ctx->join, 0), "stream wait failed");  // the schedule
   HK_CHECK(launch_step_records(ctx->model, a, rec, ctx->stream), "step records launch failed");
+  if (a.prefix) {
+    HK_CHECK(launch_decode_prefix(ctx->model, a, Q, const_cast<_Float16*>(a.Qh), e.scratch.msg, ctx->stream),
+             "prefix decode failed");
+    if ((st = table()) != HKBS_OK) return st;
+  }
   if (ctx->timing) HK_CHECK(hipEventRecord(ctx->ev[2], ctx->stream), "event record failed");
   HK_CHECK(launch_decode(ctx->model, a, ctx->stream, team), "decode launch failed");
   if (ctx->timing) {
@@ -1259,9 +1278,14 @@ hkbs_status hkbs_pmpnn_design(hkbs_pmpnn* ctx, const float* coords, const uint8_
   hipStream_t s = ctx->stream;
   HK_CHECK(hipMemcpyAsync(d_orders, host_orders.data(), norders * 4, hipMemcpyHostToDevice, s), "H2D failed");
   HK_CHECK(hipMemcpyAsync(d_seeds, sampler_seeds, (size_t)B * 8, hipMemcpyHostToDevice, s), "H2D failed");
+  bool keeps = false;  // some order starts with a residue that is not sampled
+  for (size_t q = 0; chain_mask && q < (shared ? 1 : (size_t)B); ++q) {
+    const int32_t t = host_orders[q * L];
+    keeps = keeps || chain_mask[t] * rmask[t] == 0.0F;
+  }
   if ((st = design_on_device(ctx, in.coords, in.src, in.resid, in.chain, in.chain_mask, in.true_tokens, L, B, d_orders,
                              shared, d_seeds, temperature, greedy, d_tokens, log_probs ? d_lp : nullptr,
-                             d_scores, ar, d_chosen, l0table)) != HKBS_OK)
+                             d_scores, ar, d_chosen, l0table, keeps)) != HKBS_OK)
     return st;
   HK_CHECK(hipMemcpyAsync(tokens, d_tokens, (size_t)B * L * 4, hipMemcpyDeviceToHost, s), "D2H failed");
   if (log_probs) HK_CHECK(hipMemcpyAsync(log_probs, d_lp, (size_t)B * L * kV * 4, hipMemcpyDeviceToHost, s), "D2H failed");

@@ -435,7 +435,13 @@ constexpr uint32_t kTeamAbort = 1u << 24;
 // fp32, and so do the logit weights (hi + lo, exact in fp32). In every mode
 // activations, LayerNorm, the logits (one wave per member, weights in LDS) and
 // the sampler are fp32.
-template <int PREC, int G>
+// PREFIX: one layer (a.prefix_layer) of the steps of an order's kept prefix
+// (launch_decode_prefix) instead of the pass loop: workgroup (x, y) takes steps
+// [n x, n x + n) (n = a.prefix_members) of order a.prefix_seq0 + y, whose tokens
+// are known and whose inputs of this layer earlier launches wrote, and stores
+// the layer's outputs (states and R rows, or the log-probs of the last layer)
+// with the very operations of the pass loop.
+template <int PREC, int G, bool PREFIX = false>
 __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs a) {
   constexpr bool BF = PREC == kPrecBf16, HF = PREC == kPrecFp16, X3 = PREC == kPrecBf16x3;
   constexpr bool H16 = BF || HF;        // message rows' inputs (E1, Q, R) in fp16
@@ -495,8 +501,8 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   uint16_t* const hs16 = s16 + 4 * G * kH;   // h
   uint16_t* const ffs16 = s16 + 6 * G * kH;  // ff, [hi, lo][G][kFF]
   static_assert(!M16 || G * kFF + (6 * G * kH + 2 * G * kFF) / 2 <= kPart, "16-bit staging fits part");
-  const int P = a.team;
-  int b = blockIdx.x, rank = 0;
+  const int P = PREFIX ? 1 : a.team;
+  int b = PREFIX ? a.prefix_seq0 + (int)blockIdx.y : (int)blockIdx.x, rank = 0;
   if (P > 1) {
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
     rank = slot % P;
@@ -520,10 +526,15 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   // keeps a NaN score and its tokens and log-probs are not written. Every rank
   // of a team reads the same flag, so the team leaves together.
   if (sched_meta(a.sched_tmp, L, a.shared_order ? 1 : a.B)[qo * 4 + 3] == 0) {
+    if (PREFIX) return;
     if (a.scores && rank == 0 && threadIdx.x == 0) a.scores[b] = __builtin_nanf("");
     return;
   }
-  const int npass = a.npass[qo];
+  // the order's first F steps are decoded already (launch_decode_prefix)
+  const int F = a.prefix ? a.prefix[2 * qo] : 0;
+  const int first_step = PREFIX ? (int)blockIdx.x * a.prefix_members : 0;
+  if (PREFIX && first_step >= F) return;
+  const int npass = PREFIX ? 1 : a.npass[qo];
   float* R = a.R + (size_t)b * kLayers * L * kH;
   _Float16* Rh = H16 ? a.Rh + (size_t)b * kLayers * L * kH : nullptr;  // bf16 / fp16 modes: R in fp16
   int32_t* tokens = a.tokens + (size_t)b * L;
@@ -570,14 +581,17 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   // Every token starts at -1 (not decoded yet); later passes wait for the
   // tokens of their steps' earlier neighbours (await_token) instead of for
   // the whole team.
-  if (rank == 0)
-    for (int i = threadIdx.x; i < L; i += kThreads) store_dev(tokens + i, -1);
+  if (!PREFIX && rank == 0) {
+    const int32_t* pos = a.pos + qo * L;
+    for (int i = threadIdx.x; i < L; i += kThreads)
+      if (F == 0 || pos[i] >= F) store_dev(tokens + i, -1);
+  }
   __syncthreads();
 
   // Pass 0: inactive residues (inverse_fold_scalar.cpp:804-813): fallback
   // token, zero log-probs, no draw; R rows Q + T[tok] (layer 0) and T[tok].
-  {
-    const int s0 = pstart[0], n0 = pstart[1] - pstart[0];
+  if constexpr (!PREFIX) {
+    const int s0 = pstart[0] + F, n0 = pstart[1] - s0;
     if (n0 > 0) {
       if (rank == 0) {
         for (int i = threadIdx.x; i < n0; i += kThreads) {
@@ -654,10 +668,20 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
   static_assert(kKmax % 4 == 0 && kRecFloat4 == 16 + 3 * kH / 4 && kRecRounds <= 2, "record layout");
   int ml = 0;
   if (npass >= 1) {
-    int s0 = 0;
-    ml = members(1, s0);
+    int s0 = first_step;
+    ml = PREFIX ? min(a.prefix_members, F - first_step) : members(1, s0);
 #pragma unroll
     for (int q = 0; q < kRecRounds; ++q) rec_store(ml, rec_load(s0, ml, q), q);
+  }
+  if constexpr (PREFIX) {
+    if (a.prefix_layer > 0) {  // the members' states before this layer, from the previous layer's launch
+      __syncthreads();
+      for (int task = threadIdx.x; task < ml * kH; task += kThreads) {
+        const size_t at = ((size_t)blockIdx.y * L + meta[task / kH].x) * kH + task % kH;
+        h[task] = a.prefix_h[at];
+        hA[task] = a.prefix_a[at];
+      }
+    }
   }
   if (P > 1 && !team_wait(counter, P, a.spin_limit, a.fault, &bad, a.fences)) goto finish;  // pass 0
   __builtin_amdgcn_s_waitcnt(0);  // one workgroup per sequence: its own pass-0 stores are complete
@@ -669,7 +693,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
       break;
     }
     int s0n = 0, mln = 0;  // the next pass
-    if (pass < npass) mln = members(pass + 1, s0n);
+    if (!PREFIX && pass < npass) mln = members(pass + 1, s0n);
     float4 rv[kRecRounds];
 #pragma unroll
     for (int q = 0; q < kRecRounds; ++q) rv[q] = make_float4(0.F, 0.F, 0.F, 0.F);
@@ -683,7 +707,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));  // keeps these addresses out of loop-invariant (spilled) registers
       static_assert(G * kKmax <= kThreads, "one slot per thread");
-      if (tid < ml * kKmax && tid % kKmax < K) {
+      if (!PREFIX && tid < ml * kKmax && tid % kKmax < K) {
         const int i = tid / kKmax, k = tid % kKmax;
         const int wd = nbw[tid];
         const bool bw = wd >= 0 && (wd & 0x40000000) != 0;
@@ -700,7 +724,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
       }
       __syncthreads();
       if (bad) break;
-      if (kTab && a.l0tab) {
+      if (!PREFIX && kTab && a.l0tab) {
         // x[i] = sum over slots of table rows, in the order of the MFMA path
         // below: lane group g (rows 16 mb + 4 g + e, mb outer) sums its rows,
         // then the four groups add as (g0 + g1) + (g2 + g3).
@@ -797,11 +821,12 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
       // the fp32 kernel its registers would be spilled, so there it is gathered
       // where it is used.
       constexpr bool kPrefetch = H16;
-      if (kPrefetch) gather(0, 0);
-      for (int l = 0; l < kLayers; ++l) {
+      const int l_first = PREFIX ? a.prefix_layer : 0, l_end = PREFIX ? a.prefix_layer + 1 : kLayers;
+      if (kPrefetch) gather(l_first, 0);
+      for (int l = l_first; l < l_end; ++l) {
         const DecLayerDev& w = m.dec[l];
         // Layer 0 of the fp32 and split bf16 decodes reads its message rows from the table.
-        const bool from_tab = (PREC == kPrecFp32 || X3) && l == 0 && a.l0tab != nullptr;
+        const bool from_tab = !PREFIX && (PREC == kPrecFp32 || X3) && l == 0 && a.l0tab != nullptr;
         const float* pl = prm + l * kPrmLayer;
         if (!from_tab) {  // else x holds the layer-0 message sums (table, above)
           // Message rows g1 = GELU(A + E1_tk + (bw ? R : Q)_j), two members at a time;
@@ -1047,7 +1072,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
           const bool nxt = l + 1 < kLayers;
           const DecLayerDev& nx = m.dec[nxt ? l + 1 : l];
           MDa::load(pda[0], wsel(nx.W1da_h, nx.W1da_f), nx.W1da_hl, 0, nxt ? 1 : 0);
-          if (kPrefetch && l + 1 < kLayers) gather(l + 1, 0);  // the next layer's first pair
+          if (!PREFIX && kPrefetch && l + 1 < kLayers) gather(l + 1, 0);  // the next layer's first pair
           __syncthreads();
           if (wave < ml) {
             float v[2];
@@ -1157,7 +1182,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
             GDa::load(da, (BF ? static_cast<const void*>(nx.W1da_h) : HF ? static_cast<const void*>(nx.W1da_f) : nx.W1da_t), 0,
                       nxt ? 1 : 0);
           }
-          if (kPrefetch && l + 1 < kLayers) gather(l + 1, 0);  // the next layer's first pair
+          if (!PREFIX && kPrefetch && l + 1 < kLayers) gather(l + 1, 0);  // the next layer's first pair
           __syncthreads();
           if (wave < ml) {
             float v[2];
@@ -1186,6 +1211,32 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
             }
             __syncthreads();
           }
+        }
+      }
+      if constexpr (PREFIX) {
+        // The layer's outputs (states of the next layer, its R rows); inactive residues keep their initial rows.
+        const int l = a.prefix_layer;
+        if (l + 1 < kLayers) {
+          for (int task = threadIdx.x; task < ml * kH; task += kThreads) {
+            const int t = meta[task / kH].x;
+            const size_t at = ((size_t)blockIdx.y * L + t) * kH + task % kH;
+            a.prefix_h[at] = h[task];
+            a.prefix_a[at] = hA[task];
+          }
+          constexpr int kW = H16 ? 2 : 1;  // columns per store
+          for (int task = threadIdx.x; task < ml * (kH / kW); task += kThreads) {
+            const int i = task / (kH / kW), c = kW * (task % (kH / kW));
+            const int4 mt = meta[i];
+            if (a.mask[mt.x] == 0.0F) continue;
+            const float* base = Pd + (i * 2 + l) * kH + c;
+            const float* tv = m.dec[l + 1].T + mt.w * kH + c;
+            const size_t at = ((size_t)(l + 1) * L + mt.x) * kH + c;
+            if constexpr (H16)
+              *reinterpret_cast<int32_t*>(Rh + at) = pack_h2(base[0] + tv[0], base[1] + tv[1]);
+            else
+              R[at] = base[0] + tv[0];
+          }
+          return;
         }
       }
 #pragma unroll
@@ -1228,10 +1279,16 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
         const uint64_t state = seed + (uint64_t)mt.y * 0x9E3779B97F4A7C15ull;
         const int s_tok = sample_wave(logit, T, greedy, state, &lpv);
         const int tok = __int_as_float(mt.z) == 0.0F ? mt.w : s_tok;
-        if (lp_out && lane < kV) lp_out[(size_t)t * kV + lane] = lpv;
-        if (lane == tok) store_dev(chosen + t, lpv);
-        if (lane == 0) tok_s[i] = tok;
+        if constexpr (PREFIX) {
+          float* row = a.shared_order ? a.prefix_lp : lp_out;
+          if (row && lane < kV && a.mask[t] != 0.0F) row[(size_t)t * kV + lane] = lpv;
+        } else {
+          if (lp_out && lane < kV) lp_out[(size_t)t * kV + lane] = lpv;
+          if (lane == tok) store_dev(chosen + t, lpv);
+          if (lane == 0) tok_s[i] = tok;
+        }
       }
+      if constexpr (PREFIX) return;
       __syncthreads();
       if constexpr (H16) {  // fp16 rows, two columns per device-scope store
         for (int task = threadIdx.x; task < ml * kLayers * (kH / 2); task += kThreads) {
@@ -1310,11 +1367,14 @@ finish:
 // the same LDS layout; the same MFMA operands and order; GELU(acc + b2).
 constexpr int kTabSlots = 12;  // 4 workgroups per residue: 73 us against 79 us with 24 slots at L = 300
 // Rows of slot k of residue t in the compact table: the kV token states when its
-// neighbour is decoded before t in the shared order, else its one state.
-__device__ inline int l0_slot_rows(const int32_t* __restrict__ idx, const int32_t* __restrict__ pos, int L, int K,
+// neighbour is decoded before t in the shared order, else its one state. Of an
+// order's kept prefix (its first F steps, launch_decode_prefix) a residue has
+// no rows, and as a neighbour it has one state (its Q row then holds its R row).
+__device__ inline int l0_slot_rows(const int32_t* __restrict__ idx, const int32_t* __restrict__ pos, int F, int L, int K,
                                    int t, int k) {
+  if (pos[t] < F) return 0;
   const int j = idx[(size_t)t * K + k];
-  return (j >= 0 && j < L && pos[j] < pos[t]) ? kV : 1;
+  return (j >= 0 && j < L && pos[j] < pos[t] && pos[j] >= F) ? kV : 1;
 }
 
 // Compact-table row offsets (launch_l0_rows): one workgroup; every residue's
@@ -1323,13 +1383,14 @@ __device__ inline int l0_slot_rows(const int32_t* __restrict__ idx, const int32_
 constexpr int kL0RowsThreads = 1024;
 constexpr int kL0RowsMaxL = 8192;  // the table is used while it takes <= 4 GiB: L <= 7,943
 __global__ __launch_bounds__(kL0RowsThreads) void l0_rows_kernel(const int32_t* __restrict__ idx,
-                                                                 const int32_t* __restrict__ pos, int L, int K,
+                                                                 const int32_t* __restrict__ pos, const int32_t* __restrict__ prefix, int L, int K,
                                                                  int32_t* __restrict__ base) {
   __shared__ int cnt[kL0RowsMaxL];
   __shared__ int run[kL0RowsThreads];
+  const int F = prefix ? prefix[0] : 0;
   for (int t = threadIdx.x; t < L; t += kL0RowsThreads) {
     int n = 0;
-    for (int k = 0; k < K; ++k) n += l0_slot_rows(idx, pos, L, K, t, k);
+    for (int k = 0; k < K; ++k) n += l0_slot_rows(idx, pos, F, L, K, t, k);
     cnt[t] = n;
   }
   __syncthreads();
@@ -1357,7 +1418,8 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
                                                                   const float* __restrict__ Q,
                                                                   const int32_t* __restrict__ idx,
                                                                   const int32_t* __restrict__ pos,
-                                                                  const int32_t* __restrict__ base, int L, int K,
+                                                                  const int32_t* __restrict__ base,
+                                                                  const int32_t* __restrict__ prefix, int L, int K,
                                                                   float* __restrict__ tab) {
   __shared__ __attribute__((aligned(16))) _Float16 G16[2 * kKmax * kLdH];  // hi rows, then lo rows
   __shared__ __attribute__((aligned(16))) float es[kTabSlots * kH];          // E1_tk
@@ -1371,13 +1433,15 @@ __global__ __launch_bounds__(kThreads, 4) void layer0_table_kernel(ModelDev m, c
   const int k0 = blockIdx.y * kTabSlots;
   const int nk = min(kTabSlots, K - k0);
   if (t >= L || nk <= 0) return;
+  const int F = base && prefix ? prefix[0] : 0;
+  if (base && pos[t] < F) return;
   const DecLayerDev& w = m.dec[0];
   for (int i = threadIdx.x; i < kH; i += kThreads) hA[i] = Q[((size_t)3 * L + t) * kH + i] + w.b1[i];
   if (threadIdx.x < nk) {
     const int jj = idx[(size_t)t * K + k0 + threadIdx.x];
     js[threadIdx.x] = (jj >= 0 && jj < L) ? jj : -1;
   }
-  if (threadIdx.x < K) srows[threadIdx.x] = base ? l0_slot_rows(idx, pos, L, K, t, threadIdx.x) : kL0Classes;
+  if (threadIdx.x < K) srows[threadIdx.x] = base ? l0_slot_rows(idx, pos, F, L, K, t, threadIdx.x) : kL0Classes;
   for (int i = threadIdx.x; i < kV * kH; i += kThreads) ts[i] = w.T[i];
   __syncthreads();
   if (threadIdx.x == 0) {  // exclusive running start of every slot (srows[K] = the residue's row count)
@@ -1497,6 +1561,10 @@ __global__ __launch_bounds__(128) void step_records_kernel(ModelDev m, DecodeArg
   const int32_t* order = a.shared_order ? a.orders : a.orders + (size_t)q * L;
   const int u = a.sched[(size_t)q * L + s];
   const int t = (u >= 0 && u < L) ? order[u] : -1;
+  // A neighbour in the kept prefix of a shared order counts as not decoded: its Q row holds its R row by then
+  // (launch_decode_prefix). The prefix's own steps keep their flags.
+  const int F = a.prefix && a.shared_order ? a.prefix[0] : 0;
+  const int from = u < F ? 0 : F;
   float4 v = make_float4(0.F, 0.F, 0.F, 0.F);
   if (t >= 0 && t < L) {
     if (w < kKmax / 4) {
@@ -1508,7 +1576,7 @@ __global__ __launch_bounds__(128) void step_records_kernel(ModelDev m, DecodeArg
         if (k < K) {
           const size_t at = ((size_t)q * L + u) * K + k;
           const int j = a.nbj[at];
-          if (j >= 0) wd[e] = j | (a.nbp[at] < u ? 0x40000000 : 0);
+          if (j >= 0) wd[e] = j | (a.nbp[at] < u && a.nbp[at] >= from ? 0x40000000 : 0);
         }
       }
       v = make_float4(__int_as_float(wd[0]), __int_as_float(wd[1]), __int_as_float(wd[2]), __int_as_float(wd[3]));
@@ -1520,7 +1588,7 @@ __global__ __launch_bounds__(128) void step_records_kernel(ModelDev m, DecodeArg
       uint32_t lo = 0, hi = 0;
       for (int k = 0; k < K; ++k) {
         const size_t at = ((size_t)q * L + u) * K + k;
-        if (a.nbj[at] >= 0 && a.nbp[at] < u) {
+        if (a.nbj[at] >= 0 && a.nbp[at] < u && a.nbp[at] >= from) {
           if (k < 32)
             lo |= 1u << k;
           else
@@ -1649,6 +1717,9 @@ constexpr int kSchedMaxL = 60000;  // pending counts as L bytes of LDS
 constexpr int kSchedPrioMaxL = 8192;  // balanced passes up to this length (heights, counts, frontier: 2 L bytes of LDS each)
 constexpr int kSchedCand = 1024;      // ready steps a balanced pass chooses from
 
+// Steps of order q's kept prefix, which are not scheduled (launch_decode_prefix).
+__device__ inline int sched_prefix(const int32_t* prefix, int q) { return prefix ? prefix[2 * q] : 0; }
+
 // Active step u of order q: valid residue with mask != 0.
 __device__ inline bool sched_active(const int32_t* order, const float* mask, int L, int u) {
   const int t = order[u];
@@ -1658,16 +1729,17 @@ __device__ inline bool sched_active(const int32_t* order, const float* mask, int
 // indeg[q][u]: earlier active neighbours of active step u; dcnt[q][p]: later
 // active steps that have step p as an earlier neighbour. Both zero on entry.
 __global__ void dep_count_kernel(const int32_t* __restrict__ orders, const float* __restrict__ mask,
-                                 const int32_t* __restrict__ nbp, int L, int K, int32_t* __restrict__ indeg,
-                                 int32_t* __restrict__ dcnt) {
+                                 const int32_t* __restrict__ nbp, const int32_t* __restrict__ prefix, int L, int K,
+                                 int32_t* __restrict__ indeg, int32_t* __restrict__ dcnt) {
   const int q = blockIdx.y;
+  const int F = sched_prefix(prefix, q);
   const int32_t* order = orders + (size_t)q * L;
   const int32_t* np = nbp + (size_t)q * L * K;
   const size_t n = (size_t)L * K;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     const int u = (int)(i / K);
     const int p = np[i];
-    if (p >= u || p < 0 || !sched_active(order, mask, L, u) || !sched_active(order, mask, L, p)) continue;
+    if (p >= u || p < F || !sched_active(order, mask, L, u) || !sched_active(order, mask, L, p)) continue;
     atomicAdd(indeg + (size_t)q * L + u, 1);
     atomicAdd(dcnt + (size_t)q * (L + 1) + p, 1);
   }
@@ -1697,12 +1769,14 @@ __device__ inline int block_scan(int v, int* tmp, int* total) {
   return before + inc - v;
 }
 
-// Per order (one block): permutation flag, draw indices, pass 0 (inactive
-// steps in order), exclusive offsets of the dependents lists (dcnt -> off, in
-// place, off[L] = total) and meta = {permutation, active steps, inactive steps}.
+// Per order (one block): permutation flag, draw indices, pass 0 (the kept
+// prefix, then the inactive steps, in order), exclusive offsets of the dependents lists (dcnt -> off, in
+// place, off[L] = total) and meta = {permutation, active steps after the prefix,
+// steps of pass 0}.
 __global__ __launch_bounds__(kSchedThreads) void sched_prep_kernel(const int32_t* __restrict__ orders,
                                                                    const int32_t* __restrict__ pos,
-                                                                   const float* __restrict__ mask, int L,
+                                                                   const float* __restrict__ mask,
+                                                                   const int32_t* __restrict__ prefix, int L,
                                                                    int sequential, int32_t* __restrict__ off,
                                                                    int32_t* __restrict__ draw,
                                                                    int32_t* __restrict__ sched,
@@ -1724,12 +1798,13 @@ __global__ __launch_bounds__(kSchedThreads) void sched_prep_kernel(const int32_t
   }
   __syncthreads();
   const int not_perm = bad;
+  const int F = sched_prefix(prefix, q);
   int act = 0, inact = 0, deps = 0;
   for (int u0 = 0; u0 < L; u0 += kSchedThreads) {
     const int u = u0 + threadIdx.x;
     const bool valid = u < L && order[u] >= 0 && order[u] < L;
     const bool a = valid && mask[order[u]] != 0.0F;
-    const bool z = valid && !a;
+    const bool z = valid && (!a || u < F);
     int tot;
     const int ra = block_scan(a ? 1 : 0, tmp, &tot);
     if (u < L) dq[u] = a ? act + ra : -1;
@@ -1748,7 +1823,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_prep_kernel(const int32_t
     ps[0] = 0;
     ps[1] = inact;
     meta[(size_t)q * 4 + 0] = !(not_perm || sequential);
-    meta[(size_t)q * 4 + 1] = act;
+    meta[(size_t)q * 4 + 1] = act - (prefix ? prefix[2 * q + 1] : 0);
     meta[(size_t)q * 4 + 2] = inact;
     meta[(size_t)q * 4 + 3] = !not_perm;
   }
@@ -1757,16 +1832,18 @@ __global__ __launch_bounds__(kSchedThreads) void sched_prep_kernel(const int32_t
 // dlist[q][off[p] ..]: the later active steps that wait for step p (any order
 // inside a list). cur is zero on entry.
 __global__ void dep_fill_kernel(const int32_t* __restrict__ orders, const float* __restrict__ mask,
-                                const int32_t* __restrict__ nbp, int L, int K, const int32_t* __restrict__ off,
-                                int32_t* __restrict__ cur, int32_t* __restrict__ dlist) {
+                                const int32_t* __restrict__ nbp, const int32_t* __restrict__ prefix, int L, int K,
+                                const int32_t* __restrict__ off, int32_t* __restrict__ cur,
+                                int32_t* __restrict__ dlist) {
   const int q = blockIdx.y;
+  const int F = sched_prefix(prefix, q);
   const int32_t* order = orders + (size_t)q * L;
   const int32_t* np = nbp + (size_t)q * L * K;
   const size_t n = (size_t)L * K;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     const int u = (int)(i / K);
     const int p = np[i];
-    if (p >= u || p < 0 || !sched_active(order, mask, L, u) || !sched_active(order, mask, L, p)) continue;
+    if (p >= u || p < F || !sched_active(order, mask, L, u) || !sched_active(order, mask, L, p)) continue;
     const int slot = atomicAdd(cur + (size_t)q * L + p, 1);
     dlist[(size_t)q * L * K + off[(size_t)q * (L + 1) + p] + slot] = u;
   }
@@ -1797,16 +1874,16 @@ __device__ inline uint32_t sched_ready8(const uint32_t* w, int words, int i) {
 // heights), then takes them off their own earlier neighbours' counts of
 // dependents still without one; a neighbour whose count reaches zero joins the
 // next frontier. The first frontier is every active step no step waits for.
-// ht[u] = 0xFFFF for an inactive step; outw holds the counts as 16-bit halves;
+// ht[u] = 0xFFFF for an inactive step and the F steps of the kept prefix; outw holds the counts as 16-bit halves;
 // list (nact 16-bit entries, L <= kSchedPrioMaxL) receives the frontiers one
 // after another. Returns the
 // number of rounds, the longest chain. The work is proportional to the
 // dependency pairs, not to L per round.
 __device__ int sched_heights(const int32_t* order, const float* mask, const int32_t* np, const int32_t* oq,
-                             int L, int K, uint16_t* ht, uint32_t* outw, uint16_t* list, int* tmp, int* tail) {
+                             int F, int L, int K, uint16_t* ht, uint32_t* outw, uint16_t* list, int* tmp, int* tail) {
   uint16_t* outc = reinterpret_cast<uint16_t*>(outw);
   for (int u = threadIdx.x; u < L; u += kSchedThreads) {
-    const bool a = sched_active(order, mask, L, u);
+    const bool a = u >= F && sched_active(order, mask, L, u);
     ht[u] = a ? 0 : 0xFFFF;
     outc[u] = (uint16_t)(a ? oq[u + 1] - oq[u] : 0);  // < L <= kSchedPrioMaxL
   }
@@ -1858,8 +1935,8 @@ __device__ int sched_heights(const int32_t* order, const float* mask, const int3
 //     (f forced; at most max_members): the k highest, ties to smaller u. It
 //     never defers a forced step unless max_members does.
 __global__ __launch_bounds__(kSchedThreads) void ready_schedule_kernel(
-    const int32_t* __restrict__ orders, const float* __restrict__ mask, const int32_t* __restrict__ nbp, int L,
-    int K, int max_members, int granule, const int32_t* __restrict__ indeg, const int32_t* __restrict__ off,
+    const int32_t* __restrict__ orders, const float* __restrict__ mask, const int32_t* __restrict__ nbp,
+    const int32_t* __restrict__ prefix, int L, int K, int max_members, int granule, const int32_t* __restrict__ indeg, const int32_t* __restrict__ off,
     const int32_t* __restrict__ dlist, const int32_t* __restrict__ draw, const int32_t* __restrict__ meta,
     int32_t* __restrict__ sched, int32_t* __restrict__ pstart, int32_t* __restrict__ npass) {
   // ceil(L / 4) words of pending counts, then (balanced passes) 16-bit heights
@@ -1879,11 +1956,12 @@ __global__ __launch_bounds__(kSchedThreads) void ready_schedule_kernel(
   int32_t* ps = pstart + (size_t)q * (L + 2);
   const int perm = meta[(size_t)q * 4 + 0], nact = meta[(size_t)q * 4 + 1], n0 = meta[(size_t)q * 4 + 2];
   const int32_t* dq = draw + (size_t)q * L;
+  const int F = sched_prefix(prefix, q);
   if (!perm) {
     // One pass per active step, in order of u.
     for (int u = threadIdx.x; u < L; u += kSchedThreads) {
-      const int d = dq[u];
-      if (d >= 0) {
+      const int d = dq[u] - (prefix ? prefix[2 * q + 1] : 0);
+      if (u >= F && d >= 0) {
         sq[n0 + d] = u;
         ps[1 + d + 1] = n0 + d + 1;
       }
@@ -1899,13 +1977,13 @@ __global__ __launch_bounds__(kSchedThreads) void ready_schedule_kernel(
   uint16_t* ht = reinterpret_cast<uint16_t*>(pend + words);
   int height = 0;
   if (balance)
-    height = sched_heights(order, mask, nbp + (size_t)q * L * K, oq, L, K, ht, pend + words + (L + 1) / 2,
+    height = sched_heights(order, mask, nbp + (size_t)q * L * K, oq, F, L, K, ht, pend + words + (L + 1) / 2,
                            reinterpret_cast<uint16_t*>(pend + words + 2 * ((L + 1) / 2)), tmp, &tail_s);
   for (int w = threadIdx.x; w < words; w += kSchedThreads) {
     uint32_t v = 0;
     for (int b = 0; b < 4; ++b) {
       const int u = 4 * w + b;
-      const uint32_t c = (u < L && sched_active(order, mask, L, u)) ? (uint32_t)min(ig[u], 254) : 0xFFu;
+      const uint32_t c = (u >= F && u < L && sched_active(order, mask, L, u)) ? (uint32_t)min(ig[u], 254) : 0xFFu;
       v |= c << (8 * b);
     }
     pend[w] = v;
@@ -2066,6 +2144,98 @@ __global__ __launch_bounds__(kSchedThreads) void ready_schedule_kernel(
   }
 }
 
+// Kept prefix of order q (one block): prefix[2 q] = the number of leading steps
+// before the first one that samples a token (design weight chain_mask * mask
+// != 0), 0 for an order that is not a permutation; prefix[2 q + 1] = the active
+// ones among them.
+__global__ __launch_bounds__(kSchedThreads) void prefix_steps_kernel(const int32_t* __restrict__ orders,
+                                                                     const int32_t* __restrict__ pos,
+                                                                     const float* __restrict__ mask,
+                                                                     const float* __restrict__ chain_mask, int L,
+                                                                     int32_t* __restrict__ prefix) {
+  __shared__ int first, bad, active;
+  const int q = blockIdx.x;
+  const int32_t* order = orders + (size_t)q * L;
+  if (threadIdx.x == 0) {
+    first = L;
+    bad = active = 0;
+  }
+  __syncthreads();
+  for (int u = threadIdx.x; u < L; u += kSchedThreads) {
+    const int t = order[u];
+    if (t < 0 || t >= L || pos[(size_t)q * L + t] != u)
+      bad = 1;
+    else if (chain_mask[t] * mask[t] != 0.0F)
+      atomicMin(&first, u);
+  }
+  __syncthreads();
+  const int F = bad ? 0 : first;
+  int n = 0;
+  for (int u = threadIdx.x; u < F; u += kSchedThreads) n += mask[order[u]] != 0.0F;
+  if (n) atomicAdd(&active, n);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    prefix[2 * q] = F;
+    prefix[2 * q + 1] = active;
+  }
+}
+
+// Token that a residue which is not sampled keeps: its true token, or the fallback token.
+__device__ inline int kept_token(const int32_t* true_tokens, int t) {
+  return (true_tokens && true_tokens[t] >= 0 && true_tokens[t] < kV) ? true_tokens[t] : kV - 1;
+}
+
+// Rows of the prefix steps that need no layer: block (u, y) writes step u of
+// order prefix_seq0 + y: R^0 = Q^0 + T_0[tok], for an inactive residue also
+// R^1, R^2 = T[tok] and zero log-probs (pass 0 of the decode kernel), and with
+// per-sequence orders the token.
+template <bool H16>
+__global__ __launch_bounds__(kH) void prefix_init_kernel(ModelDev m, DecodeArgs a) {
+  const int u = blockIdx.x, b = a.prefix_seq0 + blockIdx.y, c = threadIdx.x, L = a.L;
+  const size_t q = a.shared_order ? 0 : (size_t)b;
+  if (u >= a.prefix[2 * q]) return;
+  const int t = a.orders[q * L + u];
+  const int tok = kept_token(a.true_tokens, t);
+  const bool active = a.mask[t] != 0.0F;
+  for (int l = 0; l < (active ? 1 : kLayers); ++l) {
+    const float v = (l == 0 ? a.Q[(size_t)t * kH + c] : 0.0F) + m.dec[l].T[tok * kH + c];
+    const size_t at = (((size_t)b * kLayers + l) * L + t) * kH + c;
+    if constexpr (H16)
+      a.Rh[at] = static_cast<_Float16>(__builtin_amdgcn_fmed3f(v, -65504.0F, 65504.0F));
+    else
+      a.R[at] = v;
+  }
+  float* lp = a.shared_order ? a.prefix_lp : a.log_probs ? a.log_probs + (size_t)b * L * kV : nullptr;
+  if (!active && lp && c < kV) lp[(size_t)t * kV + c] = 0.0F;
+  if (!a.shared_order && c == 0) a.tokens[(size_t)b * L + t] = tok;
+}
+
+// Shared order: step u's token and log-probs to every sequence, and its R rows
+// (a.R, one sequence) in place of its Q rows, where the later steps' gathers
+// and the layer-0 table find them without knowing of the prefix.
+constexpr int kPublishSeqs = 16;  // sequences per block
+template <bool H16>
+__global__ __launch_bounds__(kH) void prefix_publish_kernel(DecodeArgs a, float* __restrict__ Q,
+                                                            _Float16* __restrict__ Qh) {
+  const int u = blockIdx.x, c = threadIdx.x, L = a.L;
+  if (u >= a.prefix[0]) return;
+  const int t = a.orders[u];
+  const int tok = kept_token(a.true_tokens, t);
+  const int b0 = blockIdx.y * kPublishSeqs, b1 = min(a.B, b0 + kPublishSeqs);
+  if (c < b1 - b0) a.tokens[(size_t)(b0 + c) * L + t] = tok;
+  if (a.log_probs)
+    for (int i = c; i < (b1 - b0) * kV; i += kH)
+      a.log_probs[((size_t)(b0 + i / kV) * L + t) * kV + i % kV] = a.prefix_lp[(size_t)t * kV + i % kV];
+  if (blockIdx.y > 0) return;
+  for (int l = 0; l < kLayers; ++l) {
+    const size_t at = ((size_t)l * L + t) * kH + c;
+    if constexpr (H16)
+      Qh[at] = a.Rh[at];
+    else
+      Q[at] = a.R[at];
+  }
+}
+
 }  // namespace
 
 hipError_t launch_positions(const int32_t* orders, int L, int n_orders, int shared, int32_t* pos, hipStream_t stream) {
@@ -2104,18 +2274,20 @@ hipError_t launch_step_records(const ModelDev& m, const DecodeArgs& a, float4* r
 }
 
 hipError_t launch_layer0_table(const ModelDev& m, const float* E1, const float* Q, const int32_t* idx,
-                               const int32_t* pos, const int32_t* base, int L, int K, float* tab, hipStream_t stream) {
+                               const int32_t* pos, const int32_t* base, const int32_t* prefix, int L, int K, float* tab,
+                               hipStream_t stream) {
   if (L <= 0 || K <= 0) return hipSuccess;
   if (K > kKmax || (base && !pos)) return hipErrorInvalidValue;
   layer0_table_kernel<<<dim3((unsigned)L, (unsigned)((K + kTabSlots - 1) / kTabSlots)), kThreads, 0, stream>>>(
-      m, E1, Q, idx, pos, base, L, K, tab);
+      m, E1, Q, idx, pos, base, prefix, L, K, tab);
   return hipGetLastError();
 }
 
-hipError_t launch_l0_rows(const int32_t* idx, const int32_t* pos, int L, int K, int32_t* base, hipStream_t stream) {
+hipError_t launch_l0_rows(const int32_t* idx, const int32_t* pos, const int32_t* prefix, int L, int K, int32_t* base,
+                          hipStream_t stream) {
   if (L <= 0 || K <= 0) return hipSuccess;
   if (K > kKmax || L > kL0RowsMaxL) return hipErrorInvalidValue;
-  l0_rows_kernel<<<1, kL0RowsThreads, 0, stream>>>(idx, pos, L, K, base);
+  l0_rows_kernel<<<1, kL0RowsThreads, 0, stream>>>(idx, pos, prefix, L, K, base);
   return hipGetLastError();
 }
 
@@ -2137,14 +2309,14 @@ hipError_t launch_decode_schedule(const DecodeArgs& a, hipStream_t stream) {
   hipError_t err = launch_zero(reinterpret_cast<float*>(indeg), nq * (3 * L + 1), stream);
   if (err != hipSuccess) return err;
   const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 2048);
-  dep_count_kernel<<<dim3(blocks, nq), 256, 0, stream>>>(a.orders, a.mask, a.nbp, a.L, a.K, indeg, off);
-  sched_prep_kernel<<<nq, kSchedThreads, 0, stream>>>(a.orders, a.pos, a.mask, a.L, sequential, off, a.draw, a.sched,
-                                                     a.pstart, meta);
-  dep_fill_kernel<<<dim3(blocks, nq), 256, 0, stream>>>(a.orders, a.mask, a.nbp, a.L, a.K, off, cur, dlist);
+  dep_count_kernel<<<dim3(blocks, nq), 256, 0, stream>>>(a.orders, a.mask, a.nbp, a.prefix, a.L, a.K, indeg, off);
+  sched_prep_kernel<<<nq, kSchedThreads, 0, stream>>>(a.orders, a.pos, a.mask, a.prefix, a.L, sequential, off, a.draw,
+                                                     a.sched, a.pstart, meta);
+  dep_fill_kernel<<<dim3(blocks, nq), 256, 0, stream>>>(a.orders, a.mask, a.nbp, a.prefix, a.L, a.K, off, cur, dlist);
   const bool balance = a.pass_granule > 1 && a.L <= kSchedPrioMaxL;
   const size_t lds_words = (L + 3) / 4 + (balance ? 3 * ((L + 1) / 2) : 0);
   ready_schedule_kernel<<<nq, kSchedThreads, sizeof(uint32_t) * lds_words, stream>>>(
-      a.orders, a.mask, a.nbp, a.L, a.K, a.max_members, a.pass_granule, indeg, off, dlist, a.draw, meta, a.sched,
+      a.orders, a.mask, a.nbp, a.prefix, a.L, a.K, a.max_members, a.pass_granule, indeg, off, dlist, a.draw, meta, a.sched,
       a.pstart, a.npass);
   return hipGetLastError();
 }
@@ -2227,6 +2399,76 @@ hipError_t launch_decode(const ModelDev& m, const DecodeArgs& args, hipStream_t 
     default:
       return launch_decode_as<kPrecFp32>(m, args, stream, max_team);
   }
+}
+
+namespace {
+
+// Prefix steps per workgroup: enough workgroups for the CUs before a second step shares one.
+constexpr int kPrefixBlocks = 256;
+
+template <int PREC>
+void launch_prefix_layer(const ModelDev& m, DecodeArgs a, int layer, int orders, hipStream_t stream) {
+  constexpr int G = decode_group(PREC, 1);
+  a.prefix_layer = layer;
+  a.prefix_members = std::max(1, std::min(G, (int)(((size_t)a.L * orders + kPrefixBlocks - 1) / kPrefixBlocks)));
+  const unsigned blocks = (unsigned)((a.L + a.prefix_members - 1) / a.prefix_members);
+  decode_kernel<PREC, G, true><<<dim3(blocks, (unsigned)orders), kThreads, 0, stream>>>(m, a);
+}
+
+}  // namespace
+
+hipError_t launch_prefix_steps(const DecodeArgs& a, hipStream_t stream) {
+  if (!a.prefix || a.L <= 0) return hipSuccess;
+  if (!a.chain_mask) return hipErrorInvalidValue;
+  prefix_steps_kernel<<<a.shared_order ? 1 : a.B, kSchedThreads, 0, stream>>>(
+      a.orders, a.pos, a.mask, a.chain_mask, a.L, const_cast<int32_t*>(a.prefix));
+  return hipGetLastError();
+}
+
+hipError_t launch_decode_prefix(const ModelDev& m, const DecodeArgs& args, float* Q, _Float16* Qh, float* scratch,
+                                hipStream_t stream) {
+  if (!args.prefix || args.L <= 0) return hipSuccess;
+  if (args.K > kKmax || args.K < kPrefixMinK) return hipErrorInvalidValue;
+  DecodeArgs a = args;
+  const bool h16 = a.precision == kPrecBf16 || a.precision == kPrecFp16;
+  const size_t LH = (size_t)a.L * kH;
+  // scratch, L (128 K + 1) floats: the states and A terms of a group of orders; a shared order's R rows and log-probs
+  const int group = a.shared_order ? 1 : std::max(1, a.K / 2);
+  a.prefix_h = scratch;
+  a.prefix_a = scratch + group * LH;
+  if (a.shared_order) {
+    a.R = scratch + 2 * LH;
+    a.Rh = reinterpret_cast<_Float16*>(a.R);
+    a.prefix_lp = scratch + 5 * LH;
+  }
+  const int nq = a.shared_order ? 1 : a.B;
+  for (int q0 = 0; q0 < nq; q0 += group) {
+    const int n = std::min(group, nq - q0);
+    a.prefix_seq0 = q0;
+    const dim3 steps((unsigned)a.L, (unsigned)n);
+    if (h16)
+      prefix_init_kernel<true><<<steps, kH, 0, stream>>>(m, a);
+    else
+      prefix_init_kernel<false><<<steps, kH, 0, stream>>>(m, a);
+    for (int l = 0; l < kLayers; ++l) {
+      if (a.precision == kPrecBf16)
+        launch_prefix_layer<kPrecBf16>(m, a, l, n, stream);
+      else if (a.precision == kPrecFp16)
+        launch_prefix_layer<kPrecFp16>(m, a, l, n, stream);
+      else if (a.precision == kPrecBf16x3 && l > 0)
+        launch_prefix_layer<kPrecBf16x3>(m, a, l, n, stream);
+      else  // split bf16 takes its layer 0 in fp32 accuracy, as its table does
+        launch_prefix_layer<kPrecFp32>(m, a, l, n, stream);
+    }
+  }
+  if (a.shared_order) {
+    const dim3 grid((unsigned)a.L, (unsigned)((a.B + kPublishSeqs - 1) / kPublishSeqs));
+    if (h16)
+      prefix_publish_kernel<true><<<grid, kH, 0, stream>>>(a, Q, Qh);
+    else
+      prefix_publish_kernel<false><<<grid, kH, 0, stream>>>(a, Q, Qh);
+  }
+  return hipGetLastError();
 }
 
 }  // namespace hkbs

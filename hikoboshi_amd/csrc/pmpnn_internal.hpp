@@ -188,6 +188,12 @@ struct DecodeArgs {
   const _Float16* E1h;    // [3][L*K][128]
   const _Float16* Qh;     // [3][L][128]: Q blocks 0..2
   _Float16* Rh;           // [B][3][L][128]
+  // Kept prefix of each order (launch_prefix_steps, launch_decode_prefix), or null: [nq][2], the leading steps that
+  // sample no token and the active ones among them. The rest is set by launch_decode_prefix for its own launches.
+  const int32_t* prefix;
+  int prefix_layer, prefix_members, prefix_seq0;
+  float *prefix_h, *prefix_a;  // [orders of a group][L][128]
+  float* prefix_lp;            // [L][21] of a shared order
 };
 // Steps one workgroup decodes in a pass, for DecodeArgs.precision and the team
 // size (workgroups per sequence): 8 in fp32 (0), where with one workgroup per
@@ -207,6 +213,18 @@ inline size_t sched_scratch_words(size_t L, size_t K, size_t nq) { return nq * (
 __host__ __device__ inline int32_t* sched_meta(int32_t* sched_tmp, size_t L, size_t nq) {
   return sched_tmp + nq * (3 * L + 1);
 }
+// Kept prefix. Random orders decode the residues that a chain mask keeps first, and until the first step that samples
+// a token nothing depends on a draw: those steps' tokens are known, so each decoder layer runs over all of them at once
+// (three launches instead of a pass per link of their dependency chain), and with a shared order they are the same in
+// every sequence and are decoded once. The rest of the decode then starts after them, with the same bits.
+// launch_prefix_steps writes a.prefix from the orders, positions and masks, before the schedule and the layer-0 table's
+// rows; launch_decode_prefix decodes the prefix after the decoder precompute and the step records and before the
+// layer-0 table: R rows, tokens and log-probs, for a shared order with the R rows in place of the prefix residues' Q
+// rows (Q, in the 16-bit modes Qh). scratch: L (128 K + 1) floats, K >= kPrefixMinK.
+constexpr int kPrefixMinK = 6;
+hipError_t launch_prefix_steps(const DecodeArgs& a, hipStream_t stream);
+hipError_t launch_decode_prefix(const ModelDev& m, const DecodeArgs& a, float* Q, _Float16* Qh, float* scratch,
+                                hipStream_t stream);
 // Per-step neighbour lists (a.nbj, a.nbp) and the pass schedule (a.sched,
 // a.pstart, a.npass, a.draw) from the orders, positions, mask and kNN graph;
 // launch_decode reads them.
@@ -248,10 +266,12 @@ hipError_t launch_q_precompute(const ModelDev& m, const float* h_v, int L, float
 constexpr int kL0Classes = kV + 1;
 inline size_t l0_table_floats(size_t L, size_t K) { return L * K * kL0Classes * kH; }
 hipError_t launch_layer0_table(const ModelDev& m, const float* E1, const float* Q, const int32_t* idx,
-                               const int32_t* pos, const int32_t* base, int L, int K, float* tab, hipStream_t stream);
+                               const int32_t* pos, const int32_t* base, const int32_t* prefix, int L, int K, float* tab,
+                               hipStream_t stream);
 // Row offsets of the compact layer-0 table of one shared order: base[t] = the
 // first row of residue t, base[L] = the row count (at most L K kV).
-hipError_t launch_l0_rows(const int32_t* idx, const int32_t* pos, int L, int K, int32_t* base, hipStream_t stream);
+hipError_t launch_l0_rows(const int32_t* idx, const int32_t* pos, const int32_t* prefix, int L, int K, int32_t* base,
+                          hipStream_t stream);
 struct TfArgs {
   const int32_t* idx;     // [L][K] global neighbour indices
   const int32_t* pos;     // [L] position of each residue in its protein's decoding order

@@ -1,0 +1,84 @@
+"""The kept prefix of a decoding order (residues that a chain mask keeps, decoded before the first sampled one) is
+decoded layer by layer instead of step by step: HKBS_DECODE_PREFIX=off leaves it to the pass loop, with the same bits
+in fp32, bf16 and fp16."""
+import numpy as np
+import pytest
+
+from hikoboshi_amd import _lib, backbone
+
+pytestmark = pytest.mark.gpu
+
+PREC = {"fp32": _lib.PRECISION_FP32, "bf16": _lib.PRECISION_BF16, "fp16": _lib.PRECISION_FP16,
+        "bf16x3": _lib.PRECISION_BF16X3}
+
+
+def _case(L, keep, seed):
+    """A backbone with residues missing atoms, a chain mask that keeps a share (an array for given residues) and true
+    tokens with entries outside the vocabulary."""
+    rng = np.random.default_rng(seed)
+    bb = backbone.single_chain(L, seed)
+    if L > 6:
+        bb.atom_sources[[2, L - 2], 0] = 0
+    mask = (rng.random(L) >= keep).astype(np.float32)
+    true = backbone.native_tokens(L, rng)
+    true[::7] = -1
+    return bb, mask, true
+
+
+def _design(ctx, bb, mask, true, B, order, monkeypatch, prefix, T=0.1):
+    monkeypatch.setenv("HKBS_DECODE_PREFIX", prefix)
+    seeds = np.arange(B, dtype=np.uint64) + 5
+    kw = {"random": dict(order_seeds=seeds),
+          "shared": dict(order_mode=_lib.ORDER_INPUT_SHARED, orders=_lib.decode_order(bb.atom_sources, 3, mask)),
+          "n_to_c": dict(order_mode=_lib.ORDER_N_TO_C)}[order]
+    return ctx.design(bb.coords, bb.atom_sources, B, seeds, temperature=T, chain_mask=mask, true_tokens=true, **kw)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("L,B,keep,order", [
+    (6, 2, 0.5, "shared"), (5, 2, 0.5, "shared"), (17, 1, 0.5, "random"), (49, 3, 0.9, "n_to_c"),
+    (130, 30, 0.7, "random"), (130, 5, 0.7, "shared"), (300, 17, 0.5, "shared"), (64, 2, 1.0, "shared"),
+    (64, 2, 1.0, "random"), (64, 2, 0.0, "shared"), (2100, 2, 0.9, "shared"),
+])
+def test_prefix_is_exact(gpu_ctx, monkeypatch, prec, L, B, keep, order):
+    bb, mask, true = _case(L, keep, 11)
+    print(f"prefix {prec} L={L} B={B} keep={keep} order={order}", flush=True)
+    gpu_ctx.set_precision(PREC[prec])
+    try:
+        on, off = (_design(gpu_ctx, bb, mask, true, B, order, monkeypatch, p) for p in ("on", "off"))
+    finally:
+        gpu_ctx.set_precision(_lib.PRECISION_FP32)
+    for key in ("tokens", "log_probs", "scores", "orders"):
+        np.testing.assert_array_equal(on[key], off[key], err_msg=key)
+
+
+@pytest.mark.parametrize("sequential", [False, True])
+def test_prefix_under_an_early_sampled_residue(gpu_ctx, monkeypatch, sequential):
+    """A sampled residue in the middle of the kept ones ends the prefix there."""
+    bb, mask, true = _case(120, 0.6, 4)
+    order = _lib.decode_order(bb.atom_sources, 9, mask)
+    kept = np.nonzero(mask == 0)[0]
+    order = np.concatenate([kept[:20], order[-1:], [r for r in order[:-1] if r not in set(kept[:20].tolist())]]).astype(np.int32)
+    if sequential:
+        monkeypatch.setenv("HKBS_DECODE_SCHEDULE", "sequential")
+    out = {}
+    for p in ("on", "off"):
+        monkeypatch.setenv("HKBS_DECODE_PREFIX", p)
+        out[p] = gpu_ctx.design(bb.coords, bb.atom_sources, 3, np.arange(3, dtype=np.uint64),
+                                order_mode=_lib.ORDER_INPUT_SHARED, orders=order, temperature=0.2, chain_mask=mask,
+                                true_tokens=true)
+    for key in ("tokens", "log_probs", "scores"):
+        np.testing.assert_array_equal(out["on"][key], out["off"][key], err_msg=key)
+
+
+def test_prefix_split_bf16(gpu_ctx, monkeypatch):
+    """Split bf16 takes the prefix's layer 0 in fp32 accuracy; nothing sampled, so that no tie can turn. Both sides
+    are within 2e-3 of fp32 at T = 0.1 (the mode's measured error), hence within 4e-3 of each other."""
+    bb, mask, true = _case(200, 1.0, 8)
+    gpu_ctx.set_precision(_lib.PRECISION_BF16X3)
+    try:
+        on, off = (_design(gpu_ctx, bb, mask, true, 2, "shared", monkeypatch, p) for p in ("on", "off"))
+    finally:
+        gpu_ctx.set_precision(_lib.PRECISION_FP32)
+    np.testing.assert_array_equal(on["tokens"], off["tokens"])
+    assert np.abs(on["log_probs"] - off["log_probs"]).max() <= 4e-3
