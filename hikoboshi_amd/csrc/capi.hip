@@ -346,6 +346,19 @@ size_t pack_t(HostArena& ar, const float* W, int N, int kin, int c0, int kd, int
   return off;
 }
 
+// Inputs c0 .. c0 + kd of W [128][kin] for seq_rows_mfma: [kd / 16][8][64][4], lane l of column block cb holds
+// W[16 cb + l % 16][c0 + 16 g + 4 j + l / 16], j = 0 .. 3.
+size_t pack_kquad(HostArena& ar, const float* W, int kin, int c0, int kd) {
+  const size_t off = ar.add((size_t)kd * 128);
+  for (int g = 0; g < kd / 16; ++g)
+    for (int cb = 0; cb < 8; ++cb)
+      for (int l = 0; l < 64; ++l)
+        for (int j = 0; j < 4; ++j)
+          ar.data[off + ((size_t)(g * 8 + cb) * 64 + l) * 4 + j] =
+              W[(size_t)(16 * cb + l % 16) * kin + c0 + 16 * g + 4 * j + l / 16];
+  return off;
+}
+
 size_t copy_raw(HostArena& ar, const float* src, size_t n, size_t pad_to = 0) {
   const size_t off = ar.add(std::max(n, pad_to));
   std::memcpy(ar.data.data() + off, src, n * sizeof(float));
@@ -518,9 +531,9 @@ hkbs_status record_call_end(hkbs_pmpnn* ctx, hipStream_t s) {
 hkbs_status build_model(hkbs_pmpnn* ctx, const float* const* t) {
   HostArena ar;
   struct Off {
-    size_t pos_w, pos_b, edge_t, ne_g, ne_b, We_t, We_b, Ws;
+    size_t pos_w, pos_b, edge_q, ne_g, ne_b, We_q, We_b, Ws;
     size_t W1b_dec_p, W1d_dec_p, Wlog_t, blog, Wlog_h, Wlog_f;
-    size_t enc[kLayers][22];
+    size_t enc[kLayers][24];
     size_t dec[kLayers][24];
     size_t dec_h[kLayers][4];  // bf16 of W3_t, Win_t, Wout_t, W1da_t as MFMA B fragments (pack_k8_t)
     size_t dec_f[kLayers][4];  // fp16 of the same
@@ -530,21 +543,23 @@ hkbs_status build_model(hkbs_pmpnn* ctx, const float* const* t) {
   } o{};
   o.pos_w = copy_raw(ar, t[0], 16 * 66);
   o.pos_b = copy_raw(ar, t[1], 16);
-  o.edge_t = pack_t(ar, t[2], 128, 416, 0, 416, 128);
+  o.edge_q = pack_kquad(ar, t[2], 416, 0, 416);
   o.ne_g = copy_raw(ar, t[3], 128);
   o.ne_b = copy_raw(ar, t[4], 128);
-  o.We_t = pack_t(ar, t[5], 128, 128, 0, 128, 128);
+  o.We_q = pack_kquad(ar, t[5], 128, 0, 128);
   o.We_b = copy_raw(ar, t[6], 128);
   o.Ws = copy_raw(ar, t[7], 21 * 128);
   for (int l = 0; l < kLayers; ++l) {
     const float* const* e = t + 8 + 22 * l;
     size_t* q = o.enc[l];
-    q[0] = pack_t(ar, e[0], 128, 384, 0, 384, 128);   // W1_t
-    q[1] = pack_t(ar, e[2], 128, 128, 0, 128, 128);   // W2_t
-    q[2] = pack_t(ar, e[4], 128, 128, 0, 128, 128);   // W3_t
-    q[3] = pack_t(ar, e[6], 128, 384, 0, 384, 128);   // W11_t
-    q[4] = pack_t(ar, e[8], 128, 128, 0, 128, 128);   // W12_t
-    q[5] = pack_t(ar, e[10], 128, 128, 0, 128, 128);  // W13_t
+    q[0] = pack_t(ar, e[0], 128, 384, 0, 128, 128);   // W1_t
+    q[1] = pack_kquad(ar, e[2], 128, 0, 128);         // W2_q
+    q[2] = pack_kquad(ar, e[4], 128, 0, 128);         // W3_q
+    q[3] = pack_t(ar, e[6], 128, 384, 0, 128, 128);   // W11_t
+    q[4] = pack_kquad(ar, e[8], 128, 0, 128);         // W12_q
+    q[5] = pack_kquad(ar, e[10], 128, 0, 128);        // W13_q
+    q[22] = pack_kquad(ar, e[0], 384, 128, 256);      // W1_q
+    q[23] = pack_kquad(ar, e[6], 384, 128, 256);      // W11_q
     q[6] = pack_t(ar, e[18], 512, 128, 0, 128, 512);  // Win_t
     q[7] = pack_t(ar, e[20], 128, 512, 0, 512, 128);  // Wout_t
     q[8] = copy_raw(ar, e[1], 128);                   // b1
@@ -668,21 +683,23 @@ hkbs_status build_model(hkbs_pmpnn* ctx, const float* const* t) {
   ModelDev& m = ctx->model;
   m.pos_w = B + o.pos_w;
   m.pos_b = B + o.pos_b;
-  m.edge_t = B + o.edge_t;
+  m.edge_q = B + o.edge_q;
   m.ne_g = B + o.ne_g;
   m.ne_b = B + o.ne_b;
-  m.We_t = B + o.We_t;
+  m.We_q = B + o.We_q;
   m.We_b = B + o.We_b;
   m.Ws = B + o.Ws;
   for (int l = 0; l < kLayers; ++l) {
     const size_t* q = o.enc[l];
     EncLayerDev& w = m.enc[l];
     w.W1_t = B + q[0];
-    w.W2_t = B + q[1];
-    w.W3_t = B + q[2];
+    w.W2_q = B + q[1];
+    w.W3_q = B + q[2];
     w.W11_t = B + q[3];
-    w.W12_t = B + q[4];
-    w.W13_t = B + q[5];
+    w.W12_q = B + q[4];
+    w.W13_q = B + q[5];
+    w.W1_q = B + q[22];
+    w.W11_q = B + q[23];
     w.Win_t = B + q[6];
     w.Wout_t = B + q[7];
     w.b1 = B + q[8];

@@ -389,6 +389,86 @@ __device__ inline void seq_gemm_mfma(float (&acc)[16], const float* A, int lda, 
   }
 }
 
+// The same sums with more waves and no weight staging (the encoder's edge
+// kernels): a wave owns 16 rows x 16 columns, and the four blocks of
+// v_mfma_f32_16x16x1_4b_f32 form four consecutive k of that block instead of
+// four column blocks of one k. A wave then has one fourth of the columns, so
+// a 16-row tile runs on eight waves (two per SIMD, whose products and adds
+// overlap) where seq_gemm_mfma ran 32 rows on four; each weight element
+// belongs to one wave, which loads it straight into registers (16 bytes per
+// lane for 16 k), so there is no LDS copy of the weights and no barrier inside
+// a product.
+//   A  : LDS tile in "k-quad" order, rows of lda floats (lda = 4 mod 32): k of
+//        a row lies at kquad(k), so that lane (row l % 16, block l / 16) reads
+//        its values of four products with one 16-byte load.
+//   W  : packed [kd / 16][8 column blocks][64 lanes][4] (pack_kquad in
+//        capi.hip): lane l's value of product j is W[16 g + 4 j + l / 16][16 cb
+//        + l % 16].
+//        Every base (W, next) is workgroup-uniform; wave cb takes block cb.
+//   ring: the weights of this product's first kQuadRing groups of 16 k, loaded
+//        by the caller (seq_ring_fill) or by the product before; this one loads
+//        the first groups of `next` (the last product: any weights) behind its
+//        own. OFF: ring slot of group 0.
+// acc[i] is output row 4 (l / 16) + i, column l % 16 of the wave's block; its
+// products are added in k order (product j, block b: k = 16 g + 4 j + b).
+constexpr int kQuadRing = 4;
+__device__ __host__ constexpr int kquad(int k) { return (k & ~15) + 4 * (k & 3) + ((k >> 2) & 3); }
+__device__ inline float4 kquad_load(const float* __restrict__ W, int g) {
+  return reinterpret_cast<const float4*>(W + (size_t)g * 2048)[threadIdx.x];
+}
+__device__ inline void seq_ring_fill(float4 (&ring)[kQuadRing], const float* __restrict__ W) {
+#pragma unroll
+  for (int d = 0; d < kQuadRing; ++d) ring[d] = kquad_load(W, d);
+}
+template <int NG, int OFF = 0>
+__device__ inline void seq_rows_mfma(float (&acc)[4], const float* A, int lda, const float* __restrict__ W,
+                                     float4 (&ring)[kQuadRing], const float* __restrict__ next) {
+#pragma clang fp contract(off)
+  static_assert(NG >= kQuadRing, "ring");
+  const int lane = threadIdx.x & 63;
+  const float* ap = A + (lane & 15) * lda + 4 * (lane >> 4);
+  const floatx16 zero = {};
+  float4 a = *reinterpret_cast<const float4*>(ap);
+  // One group of 16 k: its four products, the loads of later groups (ring slot from `from`), then its adds. Kept
+  // whole: products hoisted over other groups' adds (64 registers a group) would be spilled, and the other waves of
+  // the SIMD fill the wait for them.
+  auto group = [&](int g, float4& slot, const float* from, int fg) {
+    const float4 w = slot;
+    floatx16 p0 = __builtin_amdgcn_mfma_f32_16x16x1f32(a.x, w.x, zero, 0, 0, 0);
+    floatx16 p1 = __builtin_amdgcn_mfma_f32_16x16x1f32(a.y, w.y, zero, 0, 0, 0);
+    const float az = a.z, aw = a.w;
+    slot = kquad_load(from, fg);
+    a = *reinterpret_cast<const float4*>(ap + 16 * (g + 1 < NG ? g + 1 : g));
+    const auto add = [&](const floatx16& p) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = acc[i] + p[4 * b + i];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[i]));  // the adds are done here
+    };
+    add(p0);
+    p0 = __builtin_amdgcn_mfma_f32_16x16x1f32(az, w.z, zero, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    add(p1);
+    p1 = __builtin_amdgcn_mfma_f32_16x16x1f32(aw, w.w, zero, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    add(p0);
+    add(p1);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Groups whose ring slot refills from this product, then the last kQuadRing, which refill from the next one.
+  constexpr int kOwn = NG - kQuadRing, kLoop = kOwn / kQuadRing * kQuadRing;
+#pragma unroll 1
+  for (int g0 = 0; g0 < kLoop; g0 += kQuadRing) {
+#pragma unroll
+    for (int d = 0; d < kQuadRing; ++d) group(g0 + d, ring[(OFF + d) % kQuadRing], W, g0 + d + kQuadRing);
+  }
+#pragma unroll
+  for (int g = kLoop; g < NG; ++g)
+    group(g, ring[(OFF + g) % kQuadRing], g < kOwn ? W : next, g < kOwn ? g + kQuadRing : g - kOwn);
+}
+
 // Welford mean and 1 / sqrt(var + eps) of 128 values x[d * ld] (a k-major
 // LDS column) in the reference's order
 // (cpp/primitives/compute/layer_norm_scalar.cpp:8-40, eps 1e-5).
@@ -408,25 +488,33 @@ __device__ inline void welford_stats_col(const float* x, int ld, float* mean_out
   *inv_out = 1.0F / sqrtf(var + 1.0e-5F);
 }
 
-// LayerNorm of the rows r < rows of a column-major LDS tile (x[d * ld + r],
-// d < 128) into out (may alias x), for rows with valid(r): thread r computes
-// row r's Welford statistics (the reference's recurrence) into stat [2 *
-// rows], then the whole block normalises the elements in parallel with the
-// reference's per-element expression. Starts and ends with a barrier.
-template <typename Valid>
-__device__ inline void ln_cols_block(const float* x, float* out, int ld, int rows, const float* __restrict__ g,
-                                     const float* __restrict__ b, float* stat, Valid valid) {
+// The same statistics of a row-major LDS row (16-byte aligned), 16 values in
+// registers ahead of the recurrence.
+__device__ inline void welford_stats_row(const float* x, float* mean_out, float* inv_out) {
 #pragma clang fp contract(off)
-  __syncthreads();
-  if ((int)threadIdx.x < rows && valid((int)threadIdx.x))
-    welford_stats_col(x + threadIdx.x, ld, stat + threadIdx.x, stat + rows + threadIdx.x);
-  __syncthreads();
-  for (int i = threadIdx.x; i < rows * 128; i += blockDim.x) {
-    const int r = i % rows, d = i / rows;
-    if (!valid(r)) continue;
-    out[d * ld + r] = (x[d * ld + r] - stat[r]) * stat[rows + r] * g[d] + b[d];
+  float mean = 0.0F, m2 = 0.0F;
+  float4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<const float4*>(x)[i];
+  for (int d0 = 0; d0 < 128; d0 += 16) {
+    const float f[16] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w,
+                         v[2].x, v[2].y, v[2].z, v[2].w, v[3].x, v[3].y, v[3].z, v[3].w};
+    if (d0 + 16 < 128) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<const float4*>(x + d0 + 16)[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float count = static_cast<float>(d0 + i + 1);
+      const float delta = f[i] - mean;
+      mean += delta / count;
+      const float delta2 = f[i] - mean;
+      m2 += delta * delta2;
+    }
   }
-  __syncthreads();
+  const float var = m2 / 128.0F;
+  *mean_out = mean;
+  *inv_out = 1.0F / sqrtf(var + 1.0e-5F);
 }
 
 // Two-pass LayerNorm statistics of a 128-float row held as 2 floats per lane

@@ -10,21 +10,19 @@
 // The encoder runs once per backbone and its outputs feed every sequence,
 // and its rounding dominates the log-prob deviation at design temperatures,
 // so every product here reproduces the reference bit for bit: sequential
-// k-order sums of rounded products (seq_gemm_mfma), Welford LayerNorm, the same
+// k-order sums of rounded products (seq_rows_mfma), Welford LayerNorm, the same
 // elementwise order. The only reuse is exact: the first 128 terms of the
 // W1 / W11 sums ([h_i] part) are the same prefix for all K edges of residue
 // i, so the node kernel computes that prefix once per residue and the edge
 // kernels continue the sum with the e_ij and h_j terms.
 //
 // Kernels per layer:
-//   edge_msg_kernel    tile of 32 edge rows: W1 (e, h_j terms), W2, W3 -> m_ij.
+//   edge_msg_kernel    tile of 16 edge rows: W1 (e, h_j terms), W2, W3 -> m_ij.
 //   node_kernel        tile of 2 to 16 residues: the masked neighbour sum of
 //                      m_ij in slot order, LN1, FFN, LN2, mask, and the W11
 //                      and next-layer W1 prefixes, its weights streamed
 //                      through a ring of register stages and LDS.
-//   edge_update_kernel tile of 32 edge rows: W11, W12, W13, residual, LN3.
-// Small tiles keep several workgroups on every CU; the weights stream through
-// LDS in double-buffered chunks.
+//   edge_update_kernel tile of 16 edge rows: W11, W12, W13, residual, LN3.
 #include <cstdlib>
 #include <utility>
 
@@ -34,81 +32,97 @@
 namespace hkbs {
 namespace {
 
-constexpr int kRows = 32;    // edge rows per tile (any rows of the [L * K] edge list)
-constexpr int kLdE = 36;     // k-major leading dimension of edge tiles
-constexpr int kKC = 32;      // weight rows staged per chunk
+// Edge tiles: 16 consecutive rows of the [L * K] edge list per workgroup of
+// eight waves, wave w producing columns [16 w, 16 w + 16) (seq_rows_mfma). The
+// adds bound them, one VALU instruction for 64 products (512 products per
+// output in a layer's two kernels each); 32-row tiles on four waves, whose
+// weights went through LDS with a barrier per 32 k, left the VALU idle most of
+// the time (one or two waves per SIMD, each waiting on its own products).
+constexpr int kRows = 16;
+constexpr int kEdgeThreads = 512;
+constexpr int kLdE2 = 2 * kH + 4;  // floats per row of the [e_ij | h_j] tile (k-quad order)
+constexpr int kLdE1 = kH + 4;      // floats per row of a 128-wide tile
 
-// Loads rows of a [*, 128] row-major matrix into a k-major LDS tile
-// A[k * lda + row] (row < n_rows, gathered through rowptr), zero elsewhere.
-template <typename RowFn>
-__device__ inline void load_kmajor(float* A, int lda, int n_tile_rows, RowFn rowptr) {
-  for (int i = threadIdx.x; i < n_tile_rows * 32; i += blockDim.x) {
-    const int row = i % n_tile_rows;
-    const int kb = i / n_tile_rows;
-    const float* src = rowptr(row);
-    float4 v = make_float4(0.F, 0.F, 0.F, 0.F);
-    if (src) v = *reinterpret_cast<const float4*>(src + 4 * kb);
-    A[(4 * kb + 0) * lda + row] = v.x;
-    A[(4 * kb + 1) * lda + row] = v.y;
-    A[(4 * kb + 2) * lda + row] = v.z;
-    A[(4 * kb + 3) * lda + row] = v.w;
+// Four consecutive inputs k0 .. k0 + 3 (k0 a multiple of 4) of a k-quad row.
+__device__ inline void put_kquad4(float* row, int k0, float4 v) {
+  float* p = row + kquad(k0);  // kquad(k0 + e) = kquad(k0) + 4 e
+  p[0] = v.x;
+  p[4] = v.y;
+  p[8] = v.z;
+  p[12] = v.w;
+}
+
+// The [e_ij | h_j] rows of the tile (zero past the edge list, and for h_j of
+// an empty slot) and each row's neighbour (-1 for none).
+__device__ inline void load_edge_rows(float* E, int* nb, const float* __restrict__ h_e, const float* __restrict__ h_v,
+                                      const int32_t* __restrict__ idx, size_t slot0, size_t S, int L) {
+  const int row = threadIdx.x >> 5, q = threadIdx.x & 31;
+  const size_t slot = slot0 + row;
+  int j = slot < S ? idx[slot] : -1;
+  if (j >= L) j = -1;
+  float4 e = make_float4(0.F, 0.F, 0.F, 0.F), h = e;
+  if (slot < S) e = *reinterpret_cast<const float4*>(h_e + slot * kH + 4 * q);
+  if (j >= 0) h = *reinterpret_cast<const float4*>(h_v + (size_t)j * kH + 4 * q);
+  put_kquad4(E + row * kLdE2, 4 * q, e);
+  put_kquad4(E + row * kLdE2, kH + 4 * q, h);
+  if (q == 0) nb[row] = j;
+}
+
+// acc = the h_i prefix of the wave's outputs (prefix column c of each row's residue).
+__device__ inline void load_prefix(float (&acc)[4], const float* __restrict__ prefix, size_t slot0, size_t S, int K,
+                                   int row0, int c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const size_t slot = slot0 + row0 + i;
+    acc[i] = slot < S ? prefix[(slot / K) * 256 + c] : 0.0F;
   }
 }
 
-// Edge messages m_ij = W3 GELU(W2 GELU(W1 [h_i, e_ij, h_j] + b1) + b2) + b3 for
-// a tile of kRows consecutive edge rows; the neighbour sum is taken in order
-// by node_kernel. The products run on the matrix cores (seq_gemm_mfma): wave w
-// owns rows [16 (w % 2), + 16) and columns [64 (w / 2), + 64) of the tile.
-__global__ __launch_bounds__(256) void edge_msg_kernel(EncLayerDev w, const float* __restrict__ h_e,
-                                                       const float* __restrict__ h_v, const int32_t* __restrict__ idx,
-                                                       const float* __restrict__ prefix, int L, int K,
-                                                       float* __restrict__ msg) {
+// GELU(acc + b) of the wave's outputs into a k-quad tile; acc = 0 for the next product.
+__device__ inline void store_gelu_kquad(float (&acc)[4], float b, float* G, int row0, int c, const float* tbl) {
 #pragma clang fp contract(off)
-  __shared__ __attribute__((aligned(16))) float A[kH * kLdE];
-  __shared__ __attribute__((aligned(16))) float Wbuf[2 * kKC * kH];
+  const int at = kquad(c);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    G[(row0 + i) * kLdE1 + at] = gelu(acc[i] + b, tbl);
+    acc[i] = 0.0F;
+  }
+}
+
+// Edge messages m_ij = W3 GELU(W2 GELU(W1 [h_i, e_ij, h_j] + b1) + b2) + b3; the
+// neighbour sum is taken in order by node_kernel.
+__global__ __launch_bounds__(kEdgeThreads, 6) void edge_msg_kernel(EncLayerDev w, const float* __restrict__ h_e,
+                                                                   const float* __restrict__ h_v,
+                                                                   const int32_t* __restrict__ idx,
+                                                                   const float* __restrict__ prefix, int L, int K,
+                                                                   float* __restrict__ msg) {
+#pragma clang fp contract(off)
+  __shared__ __attribute__((aligned(16))) float E[kRows * kLdE2];
+  __shared__ __attribute__((aligned(16))) float G[2][kRows * kLdE1];
+  __shared__ int nb[kRows];
   __shared__ float tbl[17];
-  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
   const size_t S = (size_t)L * K;
   const size_t slot0 = (size_t)blockIdx.x * kRows;
-  const int n_rows = (int)min((size_t)kRows, S - slot0);
-  const int wave = threadIdx.x >> 6;
-  const int rb = 16 * (wave & 1), cb = 64 * (wave >> 1);
-
-  float acc[16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row0 = 4 * (lane >> 4), c = 16 * wave + (lane & 15);
+  float4 ring[kQuadRing];
+  seq_ring_fill(ring, w.W1_q);
+  float acc[4];
+  load_prefix(acc, prefix, slot0, S, K, row0, 128 + c);
+  load_edge_rows(E, nb, h_e, h_v, idx, slot0, S, L);
+  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
+  __syncthreads();
+  seq_rows_mfma<16>(acc, E, kLdE2, w.W1_q, ring, w.W2_q);
+  store_gelu_kquad(acc, w.b1[c], G[0], row0, c, tbl);
+  __syncthreads();
+  seq_rows_mfma<8>(acc, G[0], kLdE1, w.W2_q, ring, w.W3_q);
+  store_gelu_kquad(acc, w.b2[c], G[1], row0, c, tbl);
+  __syncthreads();
+  seq_rows_mfma<8>(acc, G[1], kLdE1, w.W3_q, ring, w.W3_q);
+  const float b3 = w.b3[c];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v);
-    acc[v] = row < n_rows ? prefix[((slot0 + row) / K) * 256 + 128 + mfma_col(cb, v)] : 0.0F;
-  }
-  load_kmajor(A, kLdE, kRows, [&](int row) -> const float* {
-    return row < n_rows ? h_e + (slot0 + row) * kH : nullptr;
-  });
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W1_t + 128 * kH, kH, kH, Wbuf, cb);
-  load_kmajor(A, kLdE, kRows, [&](int row) -> const float* {
-    if (row >= n_rows) return nullptr;
-    const int j = idx[slot0 + row];
-    return (j >= 0 && j < L) ? h_v + (size_t)j * kH : nullptr;
-  });
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W1_t + 256 * kH, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    A[c * kLdE + row] = row < n_rows ? gelu(acc[v] + w.b1[c], tbl) : 0.0F;
-    acc[v] = 0.0F;
-  }
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W2_t, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    A[c * kLdE + row] = row < n_rows ? gelu(acc[v] + w.b2[c], tbl) : 0.0F;
-    acc[v] = 0.0F;
-  }
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W3_t, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    if (row < n_rows) msg[(slot0 + row) * kH + c] = acc[v] + w.b3[c];
-  }
+  for (int i = 0; i < 4; ++i)
+    if (slot0 + row0 + i < S) msg[(slot0 + row0 + i) * kH + c] = acc[i] + b3;
 }
 
 // The weights of the node update stream through the workgroup as 40 chunks
@@ -356,69 +370,50 @@ __global__ __launch_bounds__(kNodeThreads) void node_kernel(EncLayerDev w, const
   }
 }
 
-__global__ __launch_bounds__(256) void edge_update_kernel(EncLayerDev w, float* __restrict__ h_e,
-                                                          const float* __restrict__ h_v,
-                                                          const int32_t* __restrict__ idx,
-                                                          const float* __restrict__ prefix, int L, int K) {
+__global__ __launch_bounds__(kEdgeThreads, 6) void edge_update_kernel(EncLayerDev w, float* __restrict__ h_e,
+                                                                      const float* __restrict__ h_v,
+                                                                      const int32_t* __restrict__ idx,
+                                                                      const float* __restrict__ prefix, int L, int K) {
 #pragma clang fp contract(off)
-  __shared__ __attribute__((aligned(16))) float A[kH * kLdE];
-  __shared__ __attribute__((aligned(16))) float Wbuf[2 * kKC * kH];
+  __shared__ __attribute__((aligned(16))) float E[kRows * kLdE2];
+  __shared__ __attribute__((aligned(16))) float G[2][kRows * kLdE1];
+  __shared__ int nb[kRows];
   __shared__ float tbl[17];
-  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
+  __shared__ float mean[kRows], inv[kRows];
   const size_t S = (size_t)L * K;
   const size_t slot0 = (size_t)blockIdx.x * kRows;
-  const int n_rows = (int)min((size_t)kRows, S - slot0);
-  const int wave = threadIdx.x >> 6;
-  const int rb = 16 * (wave & 1), cb = 64 * (wave >> 1);  // this wave's block (seq_gemm_mfma)
-
-  float acc[16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row0 = 4 * (lane >> 4), c = 16 * wave + (lane & 15);
+  float4 ring[kQuadRing];
+  seq_ring_fill(ring, w.W11_q);
+  float acc[4];
+  load_prefix(acc, prefix, slot0, S, K, row0, c);
+  load_edge_rows(E, nb, h_e, h_v, idx, slot0, S, L);
+  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
+  __syncthreads();
+  seq_rows_mfma<16>(acc, E, kLdE2, w.W11_q, ring, w.W12_q);
+  store_gelu_kquad(acc, w.b11[c], G[0], row0, c, tbl);
+  __syncthreads();
+  seq_rows_mfma<8>(acc, G[0], kLdE1, w.W12_q, ring, w.W13_q);
+  store_gelu_kquad(acc, w.b12[c], G[1], row0, c, tbl);
+  __syncthreads();
+  seq_rows_mfma<8>(acc, G[1], kLdE1, w.W13_q, ring, w.W13_q);
+  // x = 1 * e + m (axpy order) as plain rows, then LN3 per valid row
+  float* X = G[0];
+  const float b13 = w.b13[c];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v);
-    acc[v] = row < n_rows ? prefix[((slot0 + row) / K) * 256 + mfma_col(cb, v)] : 0.0F;
-  }
-  load_kmajor(A, kLdE, kRows, [&](int row) -> const float* {
-    return row < n_rows ? h_e + (slot0 + row) * kH : nullptr;
-  });
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W11_t + 128 * kH, kH, kH, Wbuf, cb);
-  load_kmajor(A, kLdE, kRows, [&](int row) -> const float* {
-    if (row >= n_rows) return nullptr;
-    const int j = idx[slot0 + row];
-    return (j >= 0 && j < L) ? h_v + (size_t)j * kH : nullptr;
-  });
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W11_t + 256 * kH, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    A[c * kLdE + row] = row < n_rows ? gelu(acc[v] + w.b11[c], tbl) : 0.0F;
-    acc[v] = 0.0F;
-  }
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W12_t, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    A[c * kLdE + row] = row < n_rows ? gelu(acc[v] + w.b12[c], tbl) : 0.0F;
-    acc[v] = 0.0F;
-  }
-  seq_gemm_mfma<kH, kKC>(acc, A, kLdE, rb, w.W13_t, kH, kH, Wbuf, cb);
-  // x = 1 * e + m  (axpy order), then LN3 per valid row
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = mfma_row(rb, v), c = mfma_col(cb, v);
-    A[c * kLdE + row] = (row < n_rows) ? h_e[(slot0 + row) * kH + c] + (acc[v] + w.b13[c]) : 0.0F;
-  }
-  __shared__ float ln_stat[2 * kRows];
-  __shared__ int row_ok[kRows];
-  if (threadIdx.x < kRows) {
-    const int j = (int)threadIdx.x < n_rows ? idx[slot0 + threadIdx.x] : -1;
-    row_ok[threadIdx.x] = j >= 0 && j < L;
-  }
-  ln_cols_block(A, A, kLdE, n_rows, w.n3g, w.n3b, ln_stat, [&](int r) { return row_ok[r] != 0; });
-  for (int i = threadIdx.x; i < n_rows * kH; i += blockDim.x) {
-    const int row = i / kH, c = i % kH;
-    const int j = idx[slot0 + row];
-    if (j >= 0 && j < L) h_e[(slot0 + row) * kH + c] = A[c * kLdE + row];
-  }
+  for (int i = 0; i < 4; ++i) X[(row0 + i) * kLdE1 + c] = E[(row0 + i) * kLdE2 + kquad(c)] + (acc[i] + b13);
+  __syncthreads();
+  if (threadIdx.x < kRows) welford_stats_row(X + threadIdx.x * kLdE1, mean + threadIdx.x, inv + threadIdx.x);
+  __syncthreads();
+  const int row = threadIdx.x >> 5, q = threadIdx.x & 31;
+  if (nb[row] < 0) return;
+  const float4 x = *reinterpret_cast<const float4*>(X + row * kLdE1 + 4 * q);
+  const float4 gm = *reinterpret_cast<const float4*>(w.n3g + 4 * q), bt = *reinterpret_cast<const float4*>(w.n3b + 4 * q);
+  const float mu = mean[row], is = inv[row];
+  *reinterpret_cast<float4*>(h_e + (slot0 + row) * kH + 4 * q) =
+      make_float4((x.x - mu) * is * gm.x + bt.x, (x.y - mu) * is * gm.y + bt.y, (x.z - mu) * is * gm.z + bt.z,
+                  (x.w - mu) * is * gm.w + bt.w);
 }
 
 __global__ void zero_kernel(float* __restrict__ p, size_t n) {
@@ -459,7 +454,7 @@ hipError_t launch_encoder(const ModelDev& m, const int32_t* idx, const float* ma
   const int node_rows = encoder_node_rows(L);
   const unsigned node_tiles = (unsigned)((L + node_rows - 1) / node_rows);
   for (int l = 0; l < kLayers; ++l) {
-    edge_msg_kernel<<<edge_tiles, 256, 0, stream>>>(m.enc[l], h_e, h_v, idx, ws.prefix, L, K, ws.msg);
+    edge_msg_kernel<<<edge_tiles, kEdgeThreads, 0, stream>>>(m.enc[l], h_e, h_v, idx, ws.prefix, L, K, ws.msg);
     const float* Wnext = l + 1 < kLayers ? m.enc[l + 1].W1_t : nullptr;
     if (node_rows == 16)
       node_kernel<16><<<node_tiles, kNodeThreads, 0, stream>>>(m.enc[l], Wnext, ws.msg, idx, mask, L, K, h_v, ws.prefix);
@@ -469,7 +464,7 @@ hipError_t launch_encoder(const ModelDev& m, const int32_t* idx, const float* ma
       node_kernel<4><<<node_tiles, kNodeThreads, 0, stream>>>(m.enc[l], Wnext, ws.msg, idx, mask, L, K, h_v, ws.prefix);
     else
       node_kernel<2><<<node_tiles, kNodeThreads, 0, stream>>>(m.enc[l], Wnext, ws.msg, idx, mask, L, K, h_v, ws.prefix);
-    edge_update_kernel<<<edge_tiles, 256, 0, stream>>>(m.enc[l], h_e, h_v, idx, ws.prefix, L, K);
+    edge_update_kernel<<<edge_tiles, kEdgeThreads, 0, stream>>>(m.enc[l], h_e, h_v, idx, ws.prefix, L, K);
   }
   return hipGetLastError();
 }

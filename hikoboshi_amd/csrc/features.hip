@@ -15,8 +15,7 @@
 //             the CPU path.
 // Edge embedding (inverse_fold_scalar.cpp:236-279):
 //   h_E = W_e . LayerNorm(W_edge . f) + b_e  (W_edge has no bias),
-// fused in one kernel: a 32-slot tile of features is built in LDS (k-major),
-// multiplied by W_edge, normalised and multiplied by W_e without leaving the
+// fused in one kernel: a 16-slot tile of features is built in LDS, multiplied by W_edge, normalised and multiplied by W_e without leaving the
 // CU, all in the reference's rounding order (h_E is bit-identical).
 #include "device_math.hpp"
 #include "edge_chunk.hpp"
@@ -44,66 +43,76 @@ __global__ __launch_bounds__(256) void edge_features_kernel(ModelDev m, const fl
   for (int f = 0; f < 16; ++f) dst[f] = out[f];
 }
 
-constexpr int kTile = 32;  // edge slots per workgroup
-constexpr int kLdT = 36;   // k-major leading dimension
+constexpr int kTile = 16;  // edge slots per workgroup of eight waves, 16 output columns each
+constexpr int kTileThreads = 512;
+constexpr int kLdF = kEdgeIn + 4;  // floats per row of the features, and of a 128-wide tile (both 4 mod 32)
+constexpr int kLdX = kH + 4;
 
 // h_E = W_e . LN(W_edge . f) + b_e in the reference's rounding order
-// (sequential sums without FMA, Welford LayerNorm). The 416 features of the
-// tile are built in groups of kGroupChunks 16-feature chunks (one chunk of one
-// slot per thread) and each group is consumed by the next k-range of the
-// W_edge product, so one 128-row LDS tile serves features, the W_edge output
-// and the LayerNorm output, and three workgroups fit on a CU.
-constexpr int kGroupChunks = 8;
-__global__ __launch_bounds__(256) void edge_embed_kernel(ModelDev m, const float* __restrict__ coords,
-                                                         const uint8_t* __restrict__ src,
-                                                         const int32_t* __restrict__ resid,
-                                                         const int32_t* __restrict__ chain,
-                                                         const int32_t* __restrict__ idx, int L, int K,
-                                                         float* __restrict__ h_e) {
+// (sequential sums without FMA, Welford LayerNorm), on the encoder's edge
+// tiles (seq_rows_mfma). The tile's 16 x 26 chunks of 16 features are built in
+// one round, a chunk per thread.
+__global__ __launch_bounds__(kTileThreads, 6) void edge_embed_kernel(ModelDev m, const float* __restrict__ coords,
+                                                                     const uint8_t* __restrict__ src,
+                                                                     const int32_t* __restrict__ resid,
+                                                                     const int32_t* __restrict__ chain,
+                                                                     const int32_t* __restrict__ idx, int L, int K,
+                                                                     float* __restrict__ h_e) {
 #pragma clang fp contract(off)
-  static_assert(kGroupChunks * 16 <= kH && kGroupChunks * kTile == 256, "tile sizes");
-  __shared__ __attribute__((aligned(16))) float A[kH * kLdT];
-  __shared__ __attribute__((aligned(16))) float Wbuf[2 * 32 * kH];
+  static_assert(26 * kTile <= kTileThreads && kEdgeIn == 26 * 16 && kLdF % 32 == 4 && kLdX % 32 == 4, "tile sizes");
+  __shared__ __attribute__((aligned(16))) float F[kTile * kLdF];
+  __shared__ __attribute__((aligned(16))) float X[kTile * kLdX];
+  __shared__ float mean[kTile], inv[kTile];
   __shared__ float tbl[17];
-  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
-  __syncthreads();
   const size_t S = (size_t)L * K;
   const size_t slot0 = (size_t)blockIdx.x * kTile;
-  const int wave = threadIdx.x >> 6;
-  const int rb = 16 * (wave & 1), cb = 64 * (wave >> 1);  // this wave's block (seq_gemm_mfma)
-  const int frow = threadIdx.x % kTile, fchunk = threadIdx.x / kTile;
-  const size_t fslot = slot0 + frow;
-  const int fr = fslot < S ? static_cast<int>(fslot / K) : 0;
-  const int fj = fslot < S ? idx[fslot] : -1;
-
-  float acc[16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row0 = 4 * (lane >> 4), c = 16 * wave + (lane & 15);
+  float4 ring[kQuadRing];
+  seq_ring_fill(ring, m.edge_q);
+  if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x < 26 * kTile) {
+    const int row = threadIdx.x % kTile, chunk = threadIdx.x / kTile;
+    const size_t slot = slot0 + row;
+    const int r = slot < S ? static_cast<int>(slot / K) : 0;
+    const int j = slot < S ? idx[slot] : -1;
+    float out[16];
+    edge_chunk(m, coords, src, resid, chain, L, r, j, chunk, out, tbl);  // zeros when j is not a residue
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.0F;
-  for (int c0 = 0; c0 < 26; c0 += kGroupChunks) {
-    const int nc = min(kGroupChunks, 26 - c0);
-    // A is free here: seq_gemm_mfma ends with a barrier
-    if (fchunk < nc) {
-      float out[16];
-      edge_chunk(m, coords, src, resid, chain, L, fr, fj, c0 + fchunk, out, tbl);  // zeros when fj is not a residue
-#pragma unroll
-      for (int f = 0; f < 16; ++f) A[(fchunk * 16 + f) * kLdT + frow] = out[f];
-    }
-    seq_gemm_mfma<kH, 32>(acc, A, kLdT, rb, m.edge_t + (size_t)c0 * 16 * kH, kH, nc * 16, Wbuf, cb);
+    for (int b = 0; b < 4; ++b)  // k-quad order of the chunk's 16 inputs
+      *reinterpret_cast<float4*>(F + row * kLdF + 16 * chunk + 4 * b) =
+          make_float4(out[b], out[4 + b], out[8 + b], out[12 + b]);
   }
-  float* X = A;
+  __syncthreads();
+  float acc[4] = {0.0F, 0.0F, 0.0F, 0.0F};
+  seq_rows_mfma<kEdgeIn / 16>(acc, F, kLdF, m.edge_q, ring, m.We_q);
 #pragma unroll
-  for (int v = 0; v < 16; ++v) X[mfma_col(cb, v) * kLdT + mfma_row(rb, v)] = acc[v];
-  __shared__ float ln_stat[2 * kTile];
-  ln_cols_block(X, A, kLdT, kTile, m.ne_g, m.ne_b, ln_stat, [](int) { return true; });
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.0F;
-  seq_gemm_mfma<kH, 32>(acc, A, kLdT, rb, m.We_t, kH, kH, Wbuf, cb);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const size_t slot = slot0 + mfma_row(rb, v);
-    const int c = mfma_col(cb, v);
-    if (slot < S) h_e[slot * kH + c] = acc[v] + m.We_b[c];
+  for (int i = 0; i < 4; ++i) {
+    X[(row0 + i) * kLdX + c] = acc[i];
+    acc[i] = 0.0F;
   }
+  __syncthreads();
+  if (threadIdx.x < kTile) welford_stats_row(X + threadIdx.x * kLdX, mean + threadIdx.x, inv + threadIdx.x);
+  __syncthreads();
+  float* N = F;  // the normalised rows in k-quad order, where the features were
+  {
+    const int row = threadIdx.x >> 5, q = threadIdx.x & 31;
+    const float4 x = *reinterpret_cast<const float4*>(X + row * kLdX + 4 * q);
+    const float4 gm = *reinterpret_cast<const float4*>(m.ne_g + 4 * q), bt = *reinterpret_cast<const float4*>(m.ne_b + 4 * q);
+    const float mu = mean[row], is = inv[row];
+    float* p = N + row * kLdX + kquad(4 * q);
+    p[0] = (x.x - mu) * is * gm.x + bt.x;
+    p[4] = (x.y - mu) * is * gm.y + bt.y;
+    p[8] = (x.z - mu) * is * gm.z + bt.z;
+    p[12] = (x.w - mu) * is * gm.w + bt.w;
+  }
+  __syncthreads();
+  seq_rows_mfma<kH / 16, (kEdgeIn / 16) % kQuadRing>(acc, N, kLdX, m.We_q, ring, m.We_q);
+  const float be = m.We_b[c];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (slot0 + row0 + i < S) h_e[(slot0 + row0 + i) * kH + c] = acc[i] + be;
 }
 
 }  // namespace
@@ -123,7 +132,7 @@ hipError_t launch_edge_embed(const ModelDev& m, const float* coords, const uint8
                              float* h_e, hipStream_t stream) {
   const size_t S = (size_t)L * K;
   if (S == 0) return hipSuccess;
-  edge_embed_kernel<<<(unsigned)((S + kTile - 1) / kTile), 256, 0, stream>>>(m, coords, atom_src, resid, chain,
+  edge_embed_kernel<<<(unsigned)((S + kTile - 1) / kTile), kTileThreads, 0, stream>>>(m, coords, atom_src, resid, chain,
                                                                             idx, L, K, h_e);
   return hipGetLastError();
 }

@@ -26,13 +26,13 @@ constexpr int kTensors = 118;
 //    Wp[K/16][N][16] with Wp[kb][n][j] = W[n][16 kb + j]. One float4 load per
 //    lane per four MFMA k-steps, 1 KiB contiguous per 16 columns.
 //  * "t" (transposed) for GEMVs: Wt[K][N] = W[n][k].
+//  * "k-quad" for seq_rows_mfma (N = 128): [K/16][8][64][4], see there.
 struct EncLayerDev {
-  const float* W1_t;    // [384][128]  input order [h_i | e_ij | h_j]
-  const float* W2_t;    // [128][128]
-  const float* W3_t;    // [128][128]
-  const float* W11_t;   // [384][128]
-  const float* W12_t;   // [128][128]
-  const float* W13_t;   // [128][128]
+  const float* W1_t;    // t, [128][128]: the h_i block of [h_i | e_ij | h_j]
+  const float* W11_t;
+  const float* W1_q;    // k-quad, K = 256: the e_ij and h_j blocks
+  const float* W11_q;
+  const float *W2_q, *W3_q, *W12_q, *W13_q;  // k-quad, K = 128
   const float* Win_t;   // [128][512]
   const float* Wout_t;  // [512][128]
   const float *b1, *b2, *b3, *b11, *b12, *b13, *bin, *bout;
@@ -85,9 +85,9 @@ struct DecLayerDev {
 struct ModelDev {
   const float* pos_w;  // [16][66]
   const float* pos_b;  // [16]
-  const float* edge_t; // [416][128]
+  const float* edge_q; // k-quad, 416 -> 128
   const float *ne_g, *ne_b;
-  const float* We_t;   // [128][128]
+  const float* We_q;   // k-quad, 128 -> 128
   const float* We_b;
   const float* Ws;     // [21][128]
   EncLayerDev enc[kLayers];
