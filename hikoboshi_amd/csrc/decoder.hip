@@ -772,12 +772,13 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
         __syncthreads();
       }
 
-      // Message-row gathers of members i0, i0 + 1 in layer ll (E1_tk and the R or Q
+      // Message-row gathers of kMp members from i0 in layer ll (E1_tk and the R or Q
       // row of each slot's neighbour). Every row is known when the pass starts (R
-      // rows of earlier passes), so the first pair of layer l + 1 is gathered
-      // during layer l's LayerNorm and fused product, and its latency is hidden.
+      // rows of earlier passes), so that in the 16-bit modes the first pair of layer
+      // l + 1 is gathered during layer l's LayerNorm and fused product.
       constexpr bool kPipe = H16;
-      constexpr int kS = 2 * kKmax / 16;
+      constexpr int kMp = H16 ? 2 : 1;  // members gathered at a time
+      constexpr int kS = kMp * kKmax / 16;
       static_assert(kKmax == 48 && kThreads == 512, "row mapping");
       const int c = 4 * (threadIdx.x & 31);
       const int r0 = threadIdx.x >> 5;
@@ -789,7 +790,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
           // first, so that the row loads below issue back to back (read one
           // slot at a time, every load waited for its own LDS reads).
           int wd[kS];
-          const int t0 = meta[min(i0, G - 1)].x, t1 = meta[min(i0 + 1, G - 1)].x;
+          const int t0 = meta[min(i0, G - 1)].x, t1 = meta[min(i0 + kMp - 1, G - 1)].x;
 #pragma unroll
           for (int s = 0; s < kS; ++s) {
             const int i = i0 + s / 3, k = 16 * (s % 3) + r0;  // k < kKmax
@@ -818,8 +819,8 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
           }
       };
       // The first pair of layer l + 1 is gathered during layer l (kPrefetch); in
-      // the fp32 kernel its registers would be spilled, so there it is gathered
-      // where it is used.
+      // fp32 and split bf16 it is gathered where it is used: behind the weights in
+      // flight it came later than that (fp32 decode 2 to 5 % slower).
       constexpr bool kPrefetch = H16;
       const int l_first = PREFIX ? a.prefix_layer : 0, l_end = PREFIX ? a.prefix_layer + 1 : kLayers;
       if (kPrefetch) gather(l_first, 0);
@@ -829,15 +830,18 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
         const bool from_tab = !PREFIX && (PREC == kPrecFp32 || X3) && l == 0 && a.l0tab != nullptr;
         const float* pl = prm + l * kPrmLayer;
         if (!from_tab) {  // else x holds the layer-0 message sums (table, above)
-          // Message rows g1 = GELU(A + E1_tk + (bw ? R : Q)_j), two members at a time;
-          // rows >= K are zero. Thread owns columns c..c+3 of rows r0 + 16 s
-          // (member i0 + s / 3, slot 16 (s % 3) + r0); all gathers of a pair are
-          // issued before the first use, and the next pair's once this pair's rows
-          // are in G16, so that their latency overlaps this pair's product. In the
-          // 16-bit modes the rows of all four members fit in G16 (one 16-bit copy
-          // each); otherwise G16 holds one pair (hi and lo rows) at a time.
-          // With kPrefetch the first pair's gathers are in flight already (issued
-          // before the loop for layer 0, during the previous layer otherwise).
+          // Message rows g1 = GELU(A + E1_tk + (bw ? R : Q)_j); rows >= K are zero.
+          // Thread owns columns c..c+3 of rows r0 + 16 s (slot 16 (s % 3) + r0 of
+          // member i0 + s / 3). In the 16-bit modes the rows of all four members fit
+          // in G16 (one 16-bit copy each) and are gathered a pair at a time, the next
+          // pair during this one's product; with kPrefetch the first pair's gathers
+          // are in flight already (issued before the loop for layer 0, during the
+          // previous layer otherwise). In fp32 and split bf16 (hi and lo rows) G16
+          // holds two members, the one in the product and the next one, whose rows
+          // are formed between the product's matrix instructions: both phases then
+          // run at once, where a pair's rows and then its products left the matrix
+          // cores and the VALU idle in turn (decode 13.8 -> 13.4 ms at 1,024 x 256,
+          // 5.55 -> 5.43 ms at 181 x 4 in N-to-C order, where each pass has one member).
           if (!kPrefetch) gather(l, 0);
           // W2 fragments of this wave's 16 columns stay in registers for all members.
           const int r = lane & 15, g = lane >> 4;
@@ -857,142 +861,159 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(ModelDev m, DecodeArgs
             }
           }
           const float b2 = pl[kPrmB2 + col];
-          for (int i0 = 0; i0 < ml; i0 += 2) {
-            {
-#pragma unroll
-              for (int s = 0; s < kS; ++s) {
-                const int i = i0 + s / 3, k = 16 * (s % 3) + r0;
-                if (i < ml) {
-                  float4 ev, zv;
-                  if constexpr (H16) {
-                    ev = widen_h4(e[s]);
-                    zv = widen_h4(z[s]);
-                  } else {
-                    ev = e[s];
-                    zv = z[s];
-                  }
-                  float4 xv = *reinterpret_cast<const float4*>(hA + i * kH + c);
-                  xv.x += ev.x + zv.x;
-                  xv.y += ev.y + zv.y;
-                  xv.z += ev.z + zv.z;
-                  xv.w += ev.w + zv.w;
-                  float4 v = make_float4(gelu_exp2(xv.x), gelu_exp2(xv.y), gelu_exp2(xv.z),
-                                         gelu_exp2(xv.w));
-                  if (k >= K) v = make_float4(0.F, 0.F, 0.F, 0.F);
-                  _Float16* gh = G16 + ((kPipe ? i : (s / 3) * 2) * kKmax + k) * kLdH + c;  // 16-bit: slot = member
-                  const float vv[4] = {v.x, v.y, v.z, v.w};
-                  if constexpr (BF) {
-                    bf16x4 bv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) bv[e] = static_cast<__bf16>(vv[e]);
-                    *reinterpret_cast<bf16x4*>(gh) = bv;
-                  } else if constexpr (HF) {
-                    half4 hv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) hv[e] = static_cast<_Float16>(__builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F));
-                    *reinterpret_cast<half4*>(gh) = hv;
-                  } else if constexpr (X3) {
-                    // split for the bf16 MFMA: v = hi + lo, lo = bf16(v - hi), to about 2^-16 relative
-                    bf16x4 hv, lv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                      hv[e] = static_cast<__bf16>(vv[e]);
-                      lv[e] = static_cast<__bf16>(vv[e] - static_cast<float>(hv[e]));
-                    }
-                    *reinterpret_cast<bf16x4*>(gh) = hv;
-                    *reinterpret_cast<bf16x4*>(gh + kKmax * kLdH) = lv;
-                  } else {
-                    // split for the fp16 MFMA: v = hi + lo / 2048 to about 2^-22 relative
-                    _Float16* gl = gh + kKmax * kLdH;
-                    half4 hv, lv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                      const float cl = __builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F);
-                      hv[e] = static_cast<_Float16>(cl);
-                      lv[e] = split_lo(vv[e], hv[e]);
-                    }
-                    *reinterpret_cast<half4*>(gh) = hv;
-                    *reinterpret_cast<half4*>(gl) = lv;
-                  }
-                }
-              }
+          // row_slot: the message row of slot s of the registers (member i) into G16.
+          const auto row_slot = [&](int i, int s) {
+            const int k = 16 * (s % 3) + r0;
+            float4 ev, zv;
+            if constexpr (H16) {
+              ev = widen_h4(e[s]);
+              zv = widen_h4(z[s]);
+            } else {
+              ev = e[s];
+              zv = z[s];
             }
-            __syncthreads();
-            if (i0 + 2 < ml) gather(l, i0 + 2);
-            for (int i = i0; i < ml && i < i0 + 2; ++i) {
-              const _Float16* Gh = kPipe ? G16 + i * kKmax * kLdH : G16 + (i - i0) * 2 * kKmax * kLdH;
-              const _Float16* Gl = Gh + kKmax * kLdH;
-              // W2 product: hi.hi + (hi.lo + lo.hi) / 2048 on the fp16 MFMA, or bf16 x bf16
-              floatx4 acc[3], cor[3];
+            float4 xv = *reinterpret_cast<const float4*>(hA + i * kH + c);
+            xv.x += ev.x + zv.x;
+            xv.y += ev.y + zv.y;
+            xv.z += ev.z + zv.z;
+            xv.w += ev.w + zv.w;
+            float4 v = make_float4(gelu_exp2(xv.x), gelu_exp2(xv.y), gelu_exp2(xv.z),
+                                   gelu_exp2(xv.w));
+            if (k >= K) v = make_float4(0.F, 0.F, 0.F, 0.F);
+            _Float16* gh = G16 + ((kPipe ? i : (i & 1) * 2) * kKmax + k) * kLdH + c;  // 16-bit: slot = member
+            const float vv[4] = {v.x, v.y, v.z, v.w};
+            if constexpr (BF) {
+              bf16x4 bv;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) bv[e] = static_cast<__bf16>(vv[e]);
+              *reinterpret_cast<bf16x4*>(gh) = bv;
+            } else if constexpr (HF) {
+              half4 hv;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) hv[e] = static_cast<_Float16>(__builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F));
+              *reinterpret_cast<half4*>(gh) = hv;
+            } else if constexpr (X3) {
+              // split for the bf16 MFMA: v = hi + lo, lo = bf16(v - hi), to about 2^-16 relative
+              bf16x4 hv, lv;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                hv[e] = static_cast<__bf16>(vv[e]);
+                lv[e] = static_cast<__bf16>(vv[e] - static_cast<float>(hv[e]));
+              }
+              *reinterpret_cast<bf16x4*>(gh) = hv;
+              *reinterpret_cast<bf16x4*>(gh + kKmax * kLdH) = lv;
+            } else {
+              // split for the fp16 MFMA: v = hi + lo / 2048 to about 2^-22 relative
+              _Float16* gl = gh + kKmax * kLdH;
+              half4 hv, lv;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float cl = __builtin_amdgcn_fmed3f(vv[e], -65504.0F, 65504.0F);
+                hv[e] = static_cast<_Float16>(cl);
+                lv[e] = split_lo(vv[e], hv[e]);
+              }
+              *reinterpret_cast<half4*>(gh) = hv;
+              *reinterpret_cast<half4*>(gl) = lv;
+            }
+          };
+          // product: x[i] = sum over member i's K rows of GELU(W2 g1 + b2), rows at Gh (and Gl);
+          // between(kb) runs after the products of k-block kb are issued.
+          const auto product = [&](int i, const _Float16* Gh, auto&& between) {
+            const _Float16* Gl = Gh + kKmax * kLdH;
+            // W2 product: hi.hi + (hi.lo + lo.hi) / 2048 on the fp16 MFMA, or bf16 x bf16
+            floatx4 acc[3], cor[3];
+#pragma unroll
+            for (int mb = 0; mb < 3; ++mb) {
+              acc[mb] = floatx4{0.F, 0.F, 0.F, 0.F};
+              cor[mb] = acc[mb];
+            }
+            // A operands of k-block kb for the three row blocks, double buffered:
+            // the next block's LDS reads are issued before this block's products.
+            using AOp = typename std::conditional<BF || X3, bf16x8, half8>::type;
+            AOp ah[2][3], al[2][3];
+            auto aload = [&](int kb, int buf) {
 #pragma unroll
               for (int mb = 0; mb < 3; ++mb) {
-                acc[mb] = floatx4{0.F, 0.F, 0.F, 0.F};
-                cor[mb] = acc[mb];
+                const int at = (mb * 16 + r) * kLdH + 32 * kb + 8 * g;
+                ah[buf][mb] = *reinterpret_cast<const AOp*>(Gh + at);
+                if constexpr (PREC == kPrecFp32 || X3) al[buf][mb] = *reinterpret_cast<const AOp*>(Gl + at);
               }
-              // A operands of k-block kb for the three row blocks, double buffered:
-              // the next block's LDS reads are issued before this block's products.
-              using AOp = typename std::conditional<BF || X3, bf16x8, half8>::type;
-              AOp ah[2][3], al[2][3];
-              auto aload = [&](int kb, int buf) {
+            };
+            aload(0, 0);
 #pragma unroll
-                for (int mb = 0; mb < 3; ++mb) {
-                  const int at = (mb * 16 + r) * kLdH + 32 * kb + 8 * g;
-                  ah[buf][mb] = *reinterpret_cast<const AOp*>(Gh + at);
-                  if constexpr (PREC == kPrecFp32 || X3) al[buf][mb] = *reinterpret_cast<const AOp*>(Gl + at);
-                }
-              };
-              aload(0, 0);
+            for (int kb = 0; kb < kH / 32; ++kb) {
+              if (kb + 1 < kH / 32) aload(kb + 1, (kb + 1) & 1);
+              __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-              for (int kb = 0; kb < kH / 32; ++kb) {
-                if (kb + 1 < kH / 32) aload(kb + 1, (kb + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int mb = 0; mb < 3; ++mb) {
-                  const AOp& a0 = ah[kb & 1][mb];
-                  if constexpr (BF) {
-                    acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bb[kb], acc[mb], 0, 0, 0);
-                  } else if constexpr (X3) {
-                    acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bb[kb], acc[mb], 0, 0, 0);
-                    cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bbl[kb], cor[mb], 0, 0, 0);
-                    cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[kb & 1][mb], bb[kb], cor[mb], 0, 0, 0);
-                  } else if constexpr (HF) {
-                    acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bh[kb], acc[mb], 0, 0, 0);
-                  } else {
-                    acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bh[kb], acc[mb], 0, 0, 0);
-                    cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bl[kb], cor[mb], 0, 0, 0);
-                    cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[kb & 1][mb], bh[kb], cor[mb], 0, 0, 0);
-                  }
+              for (int mb = 0; mb < 3; ++mb) {
+                const AOp& a0 = ah[kb & 1][mb];
+                if constexpr (BF) {
+                  acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bb[kb], acc[mb], 0, 0, 0);
+                } else if constexpr (X3) {
+                  acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bb[kb], acc[mb], 0, 0, 0);
+                  cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bbl[kb], cor[mb], 0, 0, 0);
+                  cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[kb & 1][mb], bb[kb], cor[mb], 0, 0, 0);
+                } else if constexpr (HF) {
+                  acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bh[kb], acc[mb], 0, 0, 0);
+                } else {
+                  acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bh[kb], acc[mb], 0, 0, 0);
+                  cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bl[kb], cor[mb], 0, 0, 0);
+                  cor[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[kb & 1][mb], bh[kb], cor[mb], 0, 0, 0);
                 }
               }
-              if constexpr (PREC == kPrecFp32) {
-#pragma unroll
-                for (int mb = 0; mb < 3; ++mb)
-#pragma unroll
-                  for (int e = 0; e < 4; ++e) acc[mb][e] += cor[mb][e] * (1.0F / 2048.0F);
-              } else if constexpr (X3) {
-#pragma unroll
-                for (int mb = 0; mb < 3; ++mb)
-#pragma unroll
-                  for (int e = 0; e < 4; ++e) acc[mb][e] += cor[mb][e];
-              }
-              // x[i][col] = sum over the member's K rows of GELU(acc + b2)
-              float sum = 0.0F;
+              between(kb);
+            }
+            if constexpr (PREC == kPrecFp32) {
 #pragma unroll
               for (int mb = 0; mb < 3; ++mb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  const int row = mb * 16 + 4 * g + e;
-                  const float gv = gelu_exp2(acc[mb][e] + b2);
-                  sum += row < K ? gv : 0.0F;
-                }
-              sum += __shfl_xor(sum, 16, 64);
-              sum += __shfl_xor(sum, 32, 64);
-              if (lane < 16) {
-                x[i * kH + col] = sum;
-                if constexpr (M16) put_split16<PREC>(xs16 + i * kH + col, G * kH, sum);
-              }
+                for (int e = 0; e < 4; ++e) acc[mb][e] += cor[mb][e] * (1.0F / 2048.0F);
+            } else if constexpr (X3) {
+#pragma unroll
+              for (int mb = 0; mb < 3; ++mb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[mb][e] += cor[mb][e];
             }
-            if constexpr (!kPipe) __syncthreads();
+            // x[i][col] = sum over the member's K rows of GELU(acc + b2)
+            float sum = 0.0F;
+#pragma unroll
+            for (int mb = 0; mb < 3; ++mb)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int row = mb * 16 + 4 * g + e;
+                const float gv = gelu_exp2(acc[mb][e] + b2);
+                sum += row < K ? gv : 0.0F;
+              }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            if (lane < 16) {
+              x[i * kH + col] = sum;
+              if constexpr (M16) put_split16<PREC>(xs16 + i * kH + col, G * kH, sum);
+            }
+          };
+          if constexpr (kPipe) {
+            for (int i0 = 0; i0 < ml; i0 += 2) {
+#pragma unroll
+              for (int s = 0; s < kS; ++s)
+                if (i0 + s / 3 < ml) row_slot(i0 + s / 3, s);
+              __syncthreads();
+              if (i0 + 2 < ml) gather(l, i0 + 2);
+              for (int i = i0; i < ml && i < i0 + 2; ++i) product(i, G16 + i * kKmax * kLdH, [](int) {});
+            }
+          } else {
+            // Two buffers of one member's hi and lo rows: the rows of member i + 1 are formed between the products of
+            // member i (the GELUs run while the matrix cores work), and its successor is gathered behind them.
+#pragma unroll
+            for (int s = 0; s < kS; ++s) row_slot(0, s);
+            __syncthreads();
+            if (1 < ml) gather(l, 1);
+            for (int i = 0; i < ml; ++i) {
+              product(i, G16 + (i & 1) * 2 * kKmax * kLdH, [&](int kb) {
+                if (kb < kS && i + 1 < ml) row_slot(i + 1, kb);
+                if (kb == kS && i + 2 < ml) gather(l, i + 2);
+              });
+              __syncthreads();
+            }
           }
           if constexpr (kPipe) __syncthreads();
         }
