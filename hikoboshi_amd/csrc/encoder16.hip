@@ -10,10 +10,10 @@
 // biases, GELU (gelu_exp2), LayerNorm (two-pass), residuals and the neighbour sum are fp32, and h_V, h_E
 // are stored in fp32. The kNN graph comes from the exact fp32 kernel.
 //
-// Edge products (the bulk of the work) run as workgroup tiles of 48 or 64 edge
+// Edge products (the bulk of the work) run as workgroup tiles of 32 to 64 edge
 // rows and four waves: the tile's operand sits in LDS already split into fp16
 // hi / lo halves, every wave reads all of its rows and produces 32 of the 128
-// output columns, so each weight fragment streamed from L2 feeds 3 or 4 row
+// output columns, so each weight fragment streamed from L2 feeds 2 to 4 row
 // blocks (the edge embedding builds its features into such a tile in two
 // parts). The node kernel keeps 16 rows per wave with the fp32 operand split
 // as it is read (wave_gemm).
@@ -26,7 +26,7 @@
 // P[i] + P[j] (no h_j block for an empty slot).
 //
 // Kernels:
-//   edge_embed16   64 edge slots per workgroup (4 waves): 416 features ->
+//   edge_embed16   32 edge slots per workgroup (4 waves): 416 features ->
 //                  W_edge -> LN -> W_e -> h_E.
 //   per layer:
 //   edge_msg16     one residue per workgroup (up to 48 slots, 4 waves): W1 e_ij +
@@ -36,7 +36,7 @@
 //                  weights) b3, LN1(h + upd), the FFN on the MFMA (a quarter
 //                  of it per wave), LN2, mask; then the four W1 / W11 blocks
 //                  of the new h.
-//   edge_update16  64 edge slots per workgroup (4 waves): W11 e_ij + P, GELU,
+//   edge_update16  32 or 64 edge slots per workgroup (4 waves): W11 e_ij + P, GELU,
 //                  W12, GELU, W13, residual, LN3 -> h_E (valid slots).
 #include "device_math.hpp"
 #include "edge_chunk.hpp"
@@ -192,19 +192,26 @@ __device__ inline void ln_acc(floatx4 (&acc)[8], const float* __restrict__ gam, 
   }
 }
 
-// 64 consecutive edge slots per workgroup: one tile of 4 row blocks. The 416
+// 32 consecutive edge slots per workgroup: one tile of 2 row blocks. The 416
 // features are built in four parts (feature chunks 0 .. 7, 8 .. 13, 14 .. 19
 // and 20 .. 25, 16 features each), so that the split slab holds 128 inputs at
-// a time and three workgroups fit a CU.
+// a time and five workgroups fit a CU. A tile is a chain of feature parts,
+// products and barriers, so that many small ones in flight beat fewer weight
+// reads per row: against tiles of 64 rows (162 registers, three workgroups) the
+// whole 16-bit encode went from 228 to 220 us at L = 20 and from 1,052 to 1,020
+// at L = 4,000 with this kernel alone changed, and scoring 512 ragged proteins
+// (2 M slots) from 35.7 - 36.1 to 35.4 - 35.8 ms.
+constexpr int kEmbedRB = 2;
 constexpr int kEmbedChunks0 = 8;  // chunks of the first part; the other three take 6 each
 constexpr int kLdE = 16 * kEmbedChunks0 + 8;  // halves per slab row
-__global__ __launch_bounds__(kTileThreads, 3) void edge_embed16_kernel(ModelDev m, const float* __restrict__ coords,
+__global__ __launch_bounds__(kTileThreads, 5) void edge_embed16_kernel(ModelDev m, const float* __restrict__ coords,
                                                                        const uint8_t* __restrict__ src,
                                                                        const int32_t* __restrict__ resid,
                                                                        const int32_t* __restrict__ chain,
                                                                        const int32_t* __restrict__ idx, int L, int K,
                                                                        float* __restrict__ h_e) {
-  constexpr int RB = 4, R = 16 * RB;
+  constexpr int RB = kEmbedRB, R = 16 * RB;
+  constexpr int kPar = 64 / R;  // feature chunks that a wave builds at once (its lanes: kPar times the R rows)
   static_assert(kEdgeIn == 26 * 16 && kLdE >= kLdS1, "feature chunks");
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * R * kLdE];
   __shared__ float stat[4][R];
@@ -216,13 +223,13 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_embed16_kernel(ModelDev 
   // neighbour j (n), their presence bits (q: bits 0-4, n: bits 8-12; bit 16:
   // j is a residue) and the positional class. Waves 0, 1 and 2 load the three
   // parts for the row of their lane.
-  // 17 floats per row: lane = row reads one column of 64 rows, so an odd stride keeps them in distinct banks
+  // 17 floats per row: a lane reads one column of its row, so an odd stride keeps the rows in distinct banks
   __shared__ float xq[R][17], xn[R][17];
   __shared__ int info[R][2];
   __shared__ float tbl[17];
   if (threadIdx.x < 17) tbl[threadIdx.x] = kExpNegTable[threadIdx.x];
   {
-    const int row = lane;
+    const int row = lane % R;
     const long long slot = base + row;
     const bool in = slot < S_;
     const int j = in ? idx[slot] : -1;
@@ -247,12 +254,12 @@ __global__ __launch_bounds__(kTileThreads, 3) void edge_embed16_kernel(ModelDev 
   }
   __syncthreads();
   floatx4 acc[RB][2];
-  // features of chunks [c0, c0 + nc) of the tile's rows into the split slab: wave w takes chunks c0 + w,
-  // c0 + w + 4, ... (wave-uniform), its lanes the 64 rows
+  // features of chunks [c0, c0 + nc) of the tile's rows into the split slab: wave w takes kPar chunks
+  // from c0 + kPar w on, ..., its lanes the R rows of each
   auto build = [&](int c0, int nc) {
-    const int row = lane;
+    const int row = lane % R;
     const int bits = info[row][0];
-    for (int c = c0 + wave; c < c0 + nc; c += 4) {
+    for (int c = c0 + kPar * wave + lane / R; c < c0 + nc; c += 4 * kPar) {
       float out[16];
       if (!(bits >> 16)) {
 #pragma unroll
@@ -489,12 +496,13 @@ __global__ __launch_bounds__(256) void node16_kernel(EncLayerDev w, Enc16LayerDe
   }
 }
 
-// 64 consecutive edge slots per workgroup: one tile of 4 row blocks.
-__global__ __launch_bounds__(kTileThreads, 3) void edge_update16_kernel(EncLayerDev w, Enc16LayerDev w16,
+// 16 RB consecutive edge slots per workgroup: one tile of RB row blocks, 2 or 4
+// by the rule of launch_encoder16.
+template <int RB>
+__global__ __launch_bounds__(kTileThreads, RB == 2 ? 4 : 3) void edge_update16_kernel(EncLayerDev w, Enc16LayerDev w16,
                                                                      float* __restrict__ h_e,
                                                                      const int32_t* __restrict__ idx,
                                                                      const float* __restrict__ prefix, int L, int K) {
-  constexpr int RB = 4;
   __shared__ __attribute__((aligned(16))) _Float16 S[2 * 16 * RB * kLdS1];
   __shared__ float stat[4][16 * RB];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -560,10 +568,10 @@ hipError_t launch_encoder16(const ModelDev& m, const float* coords, const uint8_
   if (L <= 0) return hipSuccess;
   if (K < 1 || K > kKmax) return hipErrorInvalidValue;
   const size_t S = (size_t)L * K;
-  const unsigned tiles64 = (unsigned)((S + 63) / 64);
+  const auto tiles = [&](int rb) { return (unsigned)((S + 16 * rb - 1) / (16 * rb)); };
   hipError_t e = launch_zero(h_v, (size_t)L * kH, stream);
   if (e != hipSuccess) return e;
-  edge_embed16_kernel<<<tiles64, kTileThreads, 0, stream>>>(m, coords, atom_src, resid, chain, idx, L, K, h_e);
+  edge_embed16_kernel<<<tiles(kEmbedRB), kTileThreads, 0, stream>>>(m, coords, atom_src, resid, chain, idx, L, K, h_e);
   e = launch_zero(ws.prefix, (size_t)L * kPrefix, stream);  // layer 0: h = 0, so its W1 blocks are 0
   if (e != hipSuccess) return e;
   // [L][128] weighted GELU sums and [L] weight sums of edge_msg16 (the [S][128] + L message buffer is
@@ -577,7 +585,14 @@ hipError_t launch_encoder16(const ModelDev& m, const float* coords, const uint8_
     msg<<<(unsigned)L, kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, mask, ws.prefix, L, K, gsum);
     node16_kernel<<<(unsigned)((L + 15) / 16), 256, 0, stream>>>(m.enc[l], w16, gsum, mask, L, h_v, W1_next,
                                                                 ws.prefix);
-    edge_update16_kernel<<<tiles64, kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, ws.prefix, L, K);
+    // Edge updates in tiles of 32 rows while tiles of 64 would be no more than four rounds of the card (three
+    // workgroups per CU): there the kernel is bound by its chain of products and barriers, and twice the
+    // workgroups hide it (encode 262 -> 239 us at L = 250, 1,025 -> 1,005 at L = 4,000, 3,000 tiles). Above, half the
+    // weight reads per row count for more (512 ragged proteins, 32,000 tiles per launch: 35.6 ms with 64 rows, 36.4
+    // with 32). Rows do not depend on each other: the same bits either way.
+    const bool small = tiles(4) <= 4 * 3 * 256;
+    auto* update = small ? edge_update16_kernel<2> : edge_update16_kernel<4>;
+    update<<<tiles(small ? 2 : 4), kTileThreads, 0, stream>>>(m.enc[l], w16, h_e, idx, ws.prefix, L, K);
   }
   return hipGetLastError();
 }

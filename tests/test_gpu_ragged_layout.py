@@ -26,3 +26,18 @@ def test_short_proteins_share_a_chunk(gpu_ctx, oracle, lens):
         assert sc[i] == np.float32(one_sc)
         olp, oscore = oracle.teacher_forced(bb, tok[i])
         assert np.abs(one_lp - olp).max() <= 1e-4
+
+
+@pytest.mark.parametrize("last", [1096, 1097])
+def test_edge_update_tiles_agree(gpu_ctx, last):
+    """Scoring at the edge of the tile rule (196,608 slots, then 48 more): the batch in tiles of 32 or of 64 rows is
+    bit-identical to its proteins scored alone, which take tiles of 32 rows."""
+    lens = [1000, 1000, 1000, last]
+    parts = [backbone.single_chain(n, 50 + i) for i, n in enumerate(lens)]
+    tok = [backbone.native_tokens(n, np.random.default_rng(n + i)) for i, n in enumerate(lens)]
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    print("score", lens, flush=True)
+    lp, _ = gpu_ctx.score_batch(np.concatenate([b.coords for b in parts]),
+                                np.concatenate([b.atom_sources for b in parts]), np.concatenate(tok), off)
+    for i, bb in enumerate(parts):
+        np.testing.assert_array_equal(lp[off[i]:off[i + 1]], gpu_ctx.score(bb.coords, bb.atom_sources, tok[i])[0])
