@@ -1070,7 +1070,8 @@ hkbs_status design_on_device(hkbs_pmpnn* ctx, const float* coords, const uint8_t
   HK_CHECK(launch_decode_schedule(a, ctx->side), "decode schedule launch failed");
   HK_CHECK(hipEventRecord(ctx->join, ctx->side), "event record failed");
   if (ctx->timing) HK_CHECK(hipEventRecord(ctx->ev[1], ctx->stream), "event record failed");
-  HK_CHECK(launch_decoder_precompute(ctx->model, e.h_v, e.h_e, L, K, E1, Q, ctx->stream, const_cast<_Float16*>(a.E1h),
+  HK_CHECK(launch_decoder_precompute(ctx->model, e.h_v, e.h_e, L, K, E1, Q, ctx->stream,
+                                     ctx->precision != HKBS_PRECISION_FP32, const_cast<_Float16*>(a.E1h),
                                      const_cast<_Float16*>(a.Qh)),
            "decoder precompute failed");
   HK_CHECK(launch_zero(reinterpret_cast<float*>(sync), (size_t)B + 1, ctx->stream), "workspace clear failed");

@@ -2269,11 +2269,17 @@ hipError_t launch_positions(const int32_t* orders, int L, int n_orders, int shar
 }
 
 hipError_t launch_decoder_precompute(const ModelDev& m, const float* h_v, const float* h_e, int L, int K,
-                                     float* E1, float* Q, hipStream_t stream, _Float16* E1h, _Float16* Qh) {
+                                     float* E1, float* Q, hipStream_t stream, bool split, _Float16* E1h,
+                                     _Float16* Qh) {
   const size_t S = (size_t)L * K;
   if (S == 0) return hipSuccess;
-  rows_gemm_kernel<<<dim3((unsigned)((S + kGemmRows - 1) / kGemmRows), kLayers), 256, 0, stream>>>(
-      h_e, S, m.W1b_dec_p, kLayers * kH, E1h ? nullptr : E1, E1h, kLayers);
+  if (split) {
+    const hipError_t e = launch_edge_products16(m, h_e, L, K, E1, E1h, stream);
+    if (e != hipSuccess) return e;
+  } else {
+    rows_gemm_kernel<<<dim3((unsigned)((S + kGemmRows - 1) / kGemmRows), kLayers), 256, 0, stream>>>(
+        h_e, S, m.W1b_dec_p, kLayers * kH, E1, nullptr, 0);
+  }
   rows_gemm_kernel<<<dim3((unsigned)((L + kGemmRows - 1) / kGemmRows), kLayers + 1), 256, 0, stream>>>(
       h_v, (size_t)L, m.W1d_dec_p, (kLayers + 1) * kH, Q, Qh, kLayers);
   return hipGetLastError();

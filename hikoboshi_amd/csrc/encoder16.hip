@@ -560,7 +560,57 @@ __global__ __launch_bounds__(kTileThreads, RB == 2 ? 4 : 3) void edge_update16_k
   }
 }
 
+// E1_l = W1b_l h_E of the three decoder layers, 32 edge slots per workgroup: the
+// rows are split once and kept in LDS for all three products, so that h_E is
+// read once, and a layer's stores overlap the next one's product. Bound by the
+// 2 KB per slot that it reads and writes: 123 us at L = 4,000 (192,000 slots),
+// 3.2 TB/s. The fp32 product, one workgroup per layer and tile of 64 rows, took
+// 242 us (130 us of it are the fp32 matrix cores' own time) and read the rows
+// three times. The decode of these modes rounds far more than the split does.
+__global__ __launch_bounds__(kTileThreads, 4) void edge_products16_kernel(ModelDev m, const float* __restrict__ h_e,
+                                                                          size_t slots, float* __restrict__ E1,
+                                                                          _Float16* __restrict__ E1h) {
+  constexpr int RB = 2;
+  __shared__ __attribute__((aligned(16))) _Float16 S[2 * 16 * RB * kLdS1];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int n0 = 32 * wave;
+  const size_t base = (size_t)blockIdx.x * 16 * RB;
+  tile_rows<RB>(S, h_e, [&](int row) -> long long { return base + row < slots ? (long long)(base + row) : -1; });
+  __syncthreads();
+#pragma unroll 1
+  for (int l = 0; l < kLayers; ++l) {
+    floatx4 acc[RB][2];
+    tile_gemm<RB, kH, 3>(S, kLdS1, m.dec[l].W1b_s, n0, (size_t)kH * kH, acc);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const size_t slot = base + 16 * rb + r;
+      if (slot >= slots) continue;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const size_t at = ((size_t)l * slots + slot) * kH + n0 + 16 * nt + 4 * g;
+        const floatx4 v = acc[rb][nt];
+        if (E1h) {
+          f16x4 h;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) h[i] = static_cast<_Float16>(__builtin_amdgcn_fmed3f(v[i], -65504.0F, 65504.0F));
+          *reinterpret_cast<f16x4*>(E1h + at) = h;
+        } else {
+          *reinterpret_cast<float4*>(E1 + at) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
+
+hipError_t launch_edge_products16(const ModelDev& m, const float* h_e, int L, int K, float* E1, _Float16* E1h,
+                                  hipStream_t stream) {
+  const size_t slots = (size_t)L * K;
+  if (slots == 0) return hipSuccess;
+  edge_products16_kernel<<<(unsigned)((slots + 31) / 32), kTileThreads, 0, stream>>>(m, h_e, slots, E1, E1h);
+  return hipGetLastError();
+}
 
 hipError_t launch_encoder16(const ModelDev& m, const float* coords, const uint8_t* atom_src, const int32_t* resid,
                             const int32_t* chain, const int32_t* idx, const float* mask, int L, int K, float* h_v,

@@ -59,7 +59,7 @@ struct DecLayerDev {
   const float* W2_p;   // kpack16 128 -> 128
   const float* W2h;    // [16][128][8] fp16: W2 = W2h + W2l / 2048 (decode loop)
   const float* W2l;
-  const uint16_t* W1b_s;  // W1b [16][128][8] fp16 hi, then lo (lo follows 128 * 128 halves later): teacher forcing
+  const uint16_t* W1b_s;  // W1b [16][128][8] fp16 hi, then lo (lo follows 128 * 128 halves later)
   // bf16 copies for the bf16 decode (round to nearest even), all as MFMA B
   // fragments [inputs / 8][outputs][8] (W2 like W2h; W3, Win, Wout, W1da from
   // their t-layouts)
@@ -137,12 +137,17 @@ hipError_t launch_encoder(const ModelDev& m, const int32_t* idx, const float* ma
 hipError_t launch_encoder16(const ModelDev& m, const float* coords, const uint8_t* atom_src,
                             const int32_t* resid, const int32_t* chain, const int32_t* idx, const float* mask,
                             int L, int K, float* h_v, float* h_e, const EncoderScratch& ws, hipStream_t stream);
-// E1 = W1b h_E [3][L*K][128] and Q [4][L][128]. With E1h (the 16-bit decode
+// E1 = W1b h_E [3][L*K][128] in fp32, or clamped to fp16 in E1h when that is not
+// null, on the split-operand fp16 MFMA (about 22 significant bits).
+hipError_t launch_edge_products16(const ModelDev& m, const float* h_e, int L, int K, float* E1, _Float16* E1h,
+                                  hipStream_t stream);
+// E1 = W1b h_E [3][L*K][128] and Q [4][L][128]. With split (every mode but
+// fp32) E1 comes from launch_edge_products16. With E1h (the 16-bit decode
 // modes) E1 is written only in fp16 to E1h (E1 may be null) and Qh receives an
 // fp16 copy of Q blocks 0..2; values are clamped to the fp16 range.
 hipError_t launch_decoder_precompute(const ModelDev& m, const float* h_v, const float* h_e, int L,
-                                     int K, float* E1, float* Q, hipStream_t stream, _Float16* E1h = nullptr,
-                                     _Float16* Qh = nullptr);
+                                     int K, float* E1, float* Q, hipStream_t stream, bool split,
+                                     _Float16* E1h = nullptr, _Float16* Qh = nullptr);
 struct DecodeArgs {
   const int32_t* idx;     // [L][K]
   const float* mask;      // [L]
