@@ -304,7 +304,9 @@ __device__ inline void store_acc(const floatx4 (&acc)[MB][NB], float* C, int ldc
 // group's LDS operands are read, and both are in flight while the group's 64
 // adds run. Every thread of the 256-thread block must call it (it contains
 // barriers); it starts and ends with a barrier, so LDS writes made before the
-// call are visible and A may be overwritten after it.
+// call are visible and A may be overwritten after it. The kernels use
+// seq_rows_mfma below; this form is the device check's yardstick for the
+// matrix cores' rounding.
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 __device__ inline int mfma_row(int rb, int v) { return rb + 4 * ((threadIdx.x & 63) >> 4) + (v & 3); }
 __device__ inline int mfma_col(int cb, int v) { return cb + 16 * (v >> 2) + (threadIdx.x & 15); }
